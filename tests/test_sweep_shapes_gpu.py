@@ -1,0 +1,81 @@
+"""The sweeps' two shapes -- tiles of one cell per thread on small grids, blocks
+walking rows on large ones -- at the edges of their tiles and on both sides of the
+rule that picks them.  Everything here is add, multiply, divide and square root, so
+every comparison is bit for bit."""
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from vanguard_amd import solvers as S
+
+pytestmark = pytest.mark.gpu
+
+EULER = [1.4, 0, 25, 0.3, 0.25, 250]
+
+
+def _state(physics, ny, nx):
+    rng = np.random.default_rng(ny * 1000 + nx)
+    shape = (ny, nx)
+    if physics == "euler":
+        w = rng.uniform(-0.3, 0.3, shape + (6,))
+        w[..., 0] = rng.uniform(0.5, 1.5, shape)
+        w[..., 4] = rng.uniform(0.5, 1.5, shape)
+        w[..., 5] = rng.uniform(0.0, 1.0, shape)
+    elif physics == "mhd":
+        w = rng.uniform(-0.3, 0.3, shape + (9,))
+        w[..., 0] = rng.uniform(0.5, 1.5, shape)
+        w[..., 4] = rng.uniform(0.5, 1.5, shape)
+    else:
+        w = rng.uniform(-0.05, 0.05, shape + (17,))
+        w[..., 0] += 1.0
+        w[..., 1] += 1.0 / 1.4
+        w[..., 2:11] += np.eye(3).ravel()
+    return w
+
+
+def _gpu(physics, w, dx, order, bc, steps):
+    kw = dict(order=order, limiter=1, max_steps=steps, bc=bc)
+    if physics == "euler":
+        return S.euler_solve(w, 2, dx, 0.6, np.inf, params=S.EulerMaterialParameters(*EULER), **kw)
+    if physics == "mhd":
+        return S.mhd_solve(w, 2, dx, 0.6, np.inf, params=S.MHDMaterialParameters(5.0 / 3.0, 0.0, 0.7, 0.4), **kw)
+    return S.hpr_solve(w, 2, dx, 0.4, np.inf, params=S.HPRMaterialParameters(is_thermal=False), **kw)
+
+
+def _oracle(physics, w, dx, order, bc, steps):
+    kw = dict(order=order, dim=2, dx=dx, tfinal=np.inf, max_steps=steps, bias=0.0, limiter=1, bc=bc)
+    if physics == "euler":
+        return O.euler_solve(w, cfl=0.6, params=EULER, **kw)
+    if physics == "mhd":
+        return O.mhd_solve(w, cfl=0.6, gamma=5.0 / 3.0, ch=0.7, cp=0.4, **kw)
+    return O.hpr_solve(w, cfl=0.4, subcycles=0, params=O.hpr_params(False), **kw)
+
+
+# Output rows of a y tile: 28 (SLIC; 60 for the 64-row shape), 30 (FORCE); output
+# columns of an x tile: 60 (SLIC), 62 (FORCE); y tiles are 8 or 4 columns wide.
+@pytest.mark.parametrize("physics", ["euler", "mhd", "hpr"])
+@pytest.mark.parametrize("ny,nx", [(2, 2), (28, 60), (29, 61), (30, 62), (31, 9), (57, 121), (61, 4)])
+def test_tile_edges_match_oracle(vg_ctx, physics, ny, nx):
+    w = _state(physics, ny, nx)
+    for order in (2, 1):
+        for bc in (S.TRANSMISSIVE, S.PERIODIC):
+            r = _gpu(physics, w, 1.0 / nx, order, bc, 3)
+            ref, dts = _oracle(physics, w, 1.0 / nx, order, bc, 3)
+            O.assert_bitwise(r.dt, dts, f"{physics} {ny}x{nx} order {order} bc {bc} dt")
+            O.assert_bitwise(r.cells, ref, f"{physics} {ny}x{nx} order {order} bc {bc} state")
+
+
+@pytest.mark.parametrize("physics,ny,nx,rep", [("euler", 133, 134, 10), ("mhd", 109, 110, 10), ("hpr", 82, 83, 10)])
+def test_large_grids_take_the_walking_sweeps_with_the_same_bits(vg_ctx, physics, ny, nx, rep):
+    """A periodic state repeated over a grid beyond the small-tile rule (over 160 MB
+    read and written per sweep; FORCE 96 MB) advances as its repeated unit does: the walking
+    sweeps against the tiles."""
+    unit = _state(physics, ny, nx)
+    big = np.ascontiguousarray(np.tile(unit, (rep, rep, 1)))
+    assert 2 * big.nbytes > 160 << 20 > 2 * unit.nbytes
+    for order in (2, 1):
+        a = _gpu(physics, unit, 1.0 / nx, order, S.PERIODIC, 3)
+        b = _gpu(physics, big, 1.0 / nx, order, S.PERIODIC, 3)
+        O.assert_bitwise(b.dt, a.dt, f"{physics} order {order} dt")
+        O.assert_bitwise(b.cells, np.tile(a.cells, (rep, rep, 1)), f"{physics} order {order} state")

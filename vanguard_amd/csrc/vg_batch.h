@@ -124,7 +124,7 @@ __global__ __launch_bounds__(BS) void batch_solve_kernel(BatchArgs<P> a)
             double w[NF];
             load_prim<NF>(A, n, jj, w);
             const unsigned long long k2 =
-                row_tile<P, ORDER, MODE, BS>(m, sc, a.bias, a.limiter, w, j < n, B, n, j, 1, true, s_a, s_e);
+                line_tile<P, 0, ORDER, MODE, BS, 1>(m, sc, a.bias, a.limiter, w, j < n, B, n, j, 1, true, s_a, s_e);
             key = (k2 > key) ? k2 : key;
         }
         key = block_allreduce_max<BS>(key, s_red);   // its barriers also publish B for the next step

@@ -100,40 +100,98 @@ __global__ __launch_bounds__(256) void constant_planes_kernel(const double *__re
     }
 }
 
-// ---- y-sweep shapes and their autotuner --------------------------------------
+// ---- sweep shapes ----------------------------------------------------------------
 
-// Candidate (threads per block, rows per strip, columns per thread) of the y
-// sweep: variant 0 is Tiles<P>'s shape; 1-3 trade strip length for more
-// workgroups on small grids; 4-5 give each thread two columns (two independent
-// dependency chains per wave); 6-7 are longer strips, whose wave counts on
-// 4096-row grids (3072 and 6144 per 4096 columns) fill a device running three
-// waves per SIMD in whole rounds.
+// Whether a grid's sweeps take small tiles of one cell per thread.  A block that
+// walks rows (sweep_x_kernel with several rows, sweep_y_kernel) computes no halo
+// twice and reads whole cache lines, but runs its rows one after another: with too
+// few blocks to fill the device the sweep takes as long as one walk.  Measured per
+// sweep, x walk / x tile and y walk / y tile (EXACT SLIC): Euler 200 x 200 13.9 /
+// 5.1 us and 41.9 / 5.4 us, 1024 x 1024 39.1 / 32.3 and 49.9 / 34.9; MHD 384 x 384
+// 25.4 / 15.7 and 79.0 / 16.5, 1024 x 1024 (151 MB) 80.0 / 72.1 and 85.5 / 75.0; HPR
+// 640 x 512 (89 MB) 105.7 / 79.5 and 186.6 / 75.8.  Beyond the cache the tiles' extra
+// reads of halos and partial lines count: HPR 1024 x 1024 (285 MB) 209.6 / 235.8 and
+// 187.7 / 211.8, Euler 4096 x 4096 407 / 537 and 408 / 438.  The line is drawn at
+// the bytes one sweep reads and writes, between the two; the sweeps with little
+// arithmetic to hide the reads behind (FORCE, FAST mode) meet it earlier: FAST
+// 850 x 850 (69 MB) 29.0 / 22.5, 1531 x 1000 (147 MB) 27.8 / 31.9.
+template <class P>
+bool small_tiles(int order, int mode, int ny, int nx)
+{
+    const long long bytes = 2LL * StoredFields<P>::n * 8 * ny * nx;
+    const long long most = (order == 2 && mode == VG_MODE_EXACT) ? 160LL << 20 : 96LL << 20;
+    return bytes <= most && ny <= 65535;   // ny: one row per block in the launch's second dimension
+}
+
+// Blocks of an x sweep, and its launch.
+template <class P, int ORDER>
+dim3 x_blocks(bool tiles, int ny, int nx)
+{
+    constexpr int G = (ORDER == 2) ? 2 : 1;
+    const int bs = tiles ? 64 : Tiles<P>::bsx, rx = tiles ? 1 : Tiles<P>::rx;
+    return dim3((nx + (bs - 2 * G) - 1) / (bs - 2 * G), (ny + rx - 1) / rx);
+}
+
+template <class P, int ORDER, int MODE>
+void launch_x(hipStream_t s, bool tiles, const SweepArgs<P> &a)
+{
+    const dim3 grid = x_blocks<P, ORDER>(tiles, a.ny, a.nx);
+    if (tiles) sweep_x_kernel<P, ORDER, MODE, 64, 1><<<grid, 64, 0, s>>>(a);
+    else sweep_x_kernel<P, ORDER, MODE, Tiles<P>::bsx, Tiles<P>::rx><<<grid, Tiles<P>::bsx, 0, s>>>(a);
+}
+
+// Candidate shapes of the y sweep: variant 0 walks Tiles<P>'s strips; 1-3 trade
+// strip length for more workgroups on middling grids; 4-5 are LDS tiles of 8
+// columns by 32 or 64 rows, a cell per thread (small grids, above); 6-7 are longer
+// strips, whose wave counts on 4096-row grids (3072 and 6144 per 4096 columns) fill
+// a device running three waves per SIMD in whole rounds.
 constexpr int kYVariants = 8;
 
-template <class P, int ORDER, int MODE, int BS, int H, int CPT = 1>
-int launch_y_shape(vg_ctx *ctx, const SweepArgs<P> &a)
+template <class P, int ORDER, int MODE, int BS, int H>
+void launch_y_walk(hipStream_t s, const SweepArgs<P> &a)
 {
-    dim3 grid((a.nx + BS * CPT - 1) / (BS * CPT), (a.ny + H - 1) / H);
-    return ctx->timed(ORDER == 2 ? "sweep_y_slic" : "sweep_y_force",
-                      [&] { sweep_y_kernel<P, ORDER, MODE, BS, H, CPT><<<grid, BS, 0, ctx->stream>>>(a); });
+    dim3 grid((a.nx + BS - 1) / BS, (a.ny + H - 1) / H);
+    sweep_y_kernel<P, ORDER, MODE, BS, H><<<grid, BS, 0, s>>>(a);
+}
+
+template <class P, int ORDER, int MODE, int BS, int LW>
+void launch_y_tile(hipStream_t s, const SweepArgs<P> &a)
+{
+    constexpr int OUT = BS / LW - 2 * (ORDER == 2 ? 2 : 1);
+    dim3 grid((a.nx + LW - 1) / LW, (a.ny + OUT - 1) / OUT);
+    sweep_y_tile_kernel<P, ORDER, MODE, BS, LW><<<grid, BS, 0, s>>>(a);
+}
+
+// The shape of a grid that is not tuned: the tile where small_tiles says so.
+template <class P>
+int default_y(int order, int mode, int ny, int nx)
+{
+    return small_tiles<P>(order, mode, ny, nx) ? 4 : 0;
 }
 
 template <class P, int ORDER, int MODE>
 int launch_y(vg_ctx *ctx, int variant, const SweepArgs<P> &a)
 {
-    if constexpr (Tiles<P>::tune) {
-        switch (variant) {
-        case 1: return launch_y_shape<P, ORDER, MODE, 256, 16>(ctx, a);
-        case 2: return launch_y_shape<P, ORDER, MODE, 128, 32>(ctx, a);
-        case 3: return launch_y_shape<P, ORDER, MODE, 64, 64>(ctx, a);
-        case 4: return launch_y_shape<P, ORDER, MODE, 64, 32, 2>(ctx, a);
-        case 5: return launch_y_shape<P, ORDER, MODE, 64, 64, 2>(ctx, a);
-        case 6: return launch_y_shape<P, ORDER, MODE, 256, 86>(ctx, a);
-        case 7: return launch_y_shape<P, ORDER, MODE, 256, 43>(ctx, a);
-        default: break;
+    const hipStream_t s = ctx->stream;
+    if (a.ny > 28 * 65535) variant = 0;   // more tiles than the launch's second dimension
+    return ctx->timed(ORDER == 2 ? "sweep_y_slic" : "sweep_y_force", [&] {
+        if constexpr (Tiles<P>::tune) {
+            switch (variant) {
+            case 1: return launch_y_walk<P, ORDER, MODE, 256, 16>(s, a);
+            case 2: return launch_y_walk<P, ORDER, MODE, 128, 32>(s, a);
+            case 3: return launch_y_walk<P, ORDER, MODE, 64, 64>(s, a);
+            case 4: return launch_y_tile<P, ORDER, MODE, 256, 8>(s, a);
+            case 5: return launch_y_tile<P, ORDER, MODE, 512, 8>(s, a);
+            case 6: return launch_y_walk<P, ORDER, MODE, 256, 86>(s, a);
+            case 7: return launch_y_walk<P, ORDER, MODE, 256, 43>(s, a);
+            default: break;
+            }
+        } else {
+            // 17 fields: tiles of 4 columns by 32 rows keep three blocks in a CU's LDS
+            if (variant == 4) return launch_y_tile<P, ORDER, MODE, 128, 4>(s, a);
         }
-    }
-    return launch_y_shape<P, ORDER, MODE, Tiles<P>::bsy, Tiles<P>::hy>(ctx, a);
+        launch_y_walk<P, ORDER, MODE, Tiles<P>::bsy, Tiles<P>::hy>(s, a);
+    });
 }
 
 inline std::string tune_key(const char *phys, int order, int mode, int ny, int nx)
@@ -143,7 +201,7 @@ inline std::string tune_key(const char *phys, int order, int mode, int ny, int n
 }
 
 // Picks the y-sweep shape for a grid: the context's table when the shape was
-// tuned before; otherwise each candidate runs once to warm up and three times
+// tuned before; default_y's where nothing is tuned; otherwise each candidate runs once to warm up and three times
 // timed on the caller's grid (a.in -> a.out, with a.clk a scratch clock holding
 // a small positive dt, no CFL fusion), and the fastest is recorded.
 template <class P, int ORDER, int MODE>
@@ -154,7 +212,7 @@ int tune_y(vg_ctx *ctx, const std::string &key, SweepArgs<P> a, int &variant)
         variant = it->second;
         return VG_OK;
     }
-    variant = 0;
+    variant = default_y<P>(ORDER, MODE, a.ny, a.nx);
     if (!Tiles<P>::tune || !ctx->autotune || ctx->timing) return VG_OK;
     a.fuse_max = 0;
     hipEvent_t e0, e1;
@@ -185,8 +243,7 @@ template <class P>
 struct GridState {
     static constexpr int NF = P::NF;
     static constexpr int NS = StoredFields<P>::n;   // planes per buffer (stored fields per cell)
-    static constexpr int kBSX = Tiles<P>::bsx, kRX = Tiles<P>::rx, kBSY = Tiles<P>::bsy, kHY = Tiles<P>::hy;
-    vg_ctx *ctx = nullptr;
+        vg_ctx *ctx = nullptr;
     int dim = 2, ny = 1, nx = 1;
     long long plane = 0, cells = 0;
     double *buf[2] = {nullptr, nullptr};
@@ -202,7 +259,7 @@ struct GridState {
     int subcycles = 0;             // source sub-cycles per half step (SourceStage)
     typename P::Params last_params{};
     int last_bc = -1;
-    int y_variant = 0;             // y-sweep shape (autotuned per grid shape)
+    int y_variant = -1;            // y-sweep shape, autotuned per grid shape (-1: default_y)
     bool reduced = false;          // this run sweeps with ReducedPhys<P> (constant planes checked)
     bool planar_known = false;     // both buffers hold the constant planes (checked since the last load)
     int *flag = nullptr;           // device flag of the constant-plane check (lazy)
@@ -225,9 +282,9 @@ struct GridState {
         VG_HIP(hipMalloc(&buf[1], sizeof(double) * NS * plane));
         VG_HIP(hipMalloc(&clk, sizeof(Clock)));
         VG_HIP(hipMalloc(&scan, 2 * sizeof(unsigned long long)));
-        const long long gx = (nx + kBSX - 4 - 1) / (kBSX - 4) + 1;
-        // one per block of the largest producer: x sweep tiles, 64-cell wave-speed
-        // blocks, or the source stage's tiles of 32 x 4 cells
+        const long long gx = (nx + 64 - 4 - 1) / (64 - 4);
+        // one per block of the largest producer: x sweep tiles of 64 cells, 64-cell
+        // wave-speed blocks, or the source stage's tiles of 32 x 4 cells
         const long long tiles = (long long)((nx + 31) / 32) * ((ny + 3) / 4);
         const long long slots = std::max<long long>(std::max<long long>(gx * ny, cells / 64 + 1), std::max(tiles, 4096LL));
         VG_HIP(hipMalloc(&partials, sizeof(unsigned long long) * slots));
@@ -284,7 +341,7 @@ struct GridState {
         subcycles = o.subcycles;
         last_params = typename P::Params{};
         last_bc = -1;
-        y_variant = 0;
+        y_variant = -1;
         reduced = false;
         planar_known = false;
         flag = o.flag;
@@ -345,11 +402,12 @@ struct GridState {
 
     // Blocks of the launch that ends a step and folds in the next step's CFL
     // maximum: the last source sub-cycle, else the last x sweep.
-    int fused_count(int order) const
+    int fused_count(int order, int mode = VG_MODE_EXACT) const
     {
         if (SourceStage<P>::kActive && subcycles > 0 && order == 2) return (int)SourceStage<P>::blocks(*this);
-        const int G = (order == 2) ? 2 : 1;
-        return (int)(((nx + (kBSX - 2 * G) - 1) / (kBSX - 2 * G)) * (long long)((ny + kRX - 1) / kRX));
+        const bool tiles = small_tiles<P>(order, mode, ny, nx);
+        const dim3 g = (order == 2) ? x_blocks<P, 2>(tiles, ny, nx) : x_blocks<P, 1>(tiles, ny, nx);
+        return (int)(g.x * g.y);
     }
 
     // Wave-speed maximum of the current grid into clk->smax (and the corner
@@ -403,16 +461,14 @@ struct GridState {
         a.partials = partials;
         a.fixed_params = fixed_params;
         if (dir == 0) {
-            constexpr int G = (ORDER == 2) ? 2 : 1;
-            dim3 grid((nx + (kBSX - 2 * G) - 1) / (kBSX - 2 * G), (ny + kRX - 1) / kRX);
-            if (fuse) n_partials = (int)(grid.x * grid.y);
+            if (fuse) n_partials = fused_count(ORDER, MODE);
             return ctx->timed(ORDER == 2 ? "sweep_x_slic" : "sweep_x_force", [&] {
-                sweep_x_kernel<Q, ORDER, MODE, kBSX, kRX><<<grid, kBSX, 0, ctx->stream>>>(a);
+                launch_x<Q, ORDER, MODE>(ctx->stream, small_tiles<P>(ORDER, MODE, ny, nx), a);
             });
         }
         // The y sweep never ends a step, so it never writes the CFL partials.
         a.fuse_max = 0;
-        return launch_y<Q, ORDER, MODE>(ctx, y_variant, a);
+        return launch_y<Q, ORDER, MODE>(ctx, y_variant >= 0 ? y_variant : default_y<P>(ORDER, MODE, ny, nx), a);
     }
 
     template <int ORDER, int MODE>
@@ -534,7 +590,7 @@ struct GridState {
             // the same number of partials a fused sweep would write
             rc = PostStep<P>::launch(*this, a, m);
             if (rc) return rc;
-            wave_max_kernel<P><<<fused_count(ORDER), 256, 0, ctx->stream>>>(a, plane, cells, dim, m, partials);
+            wave_max_kernel<P><<<fused_count(ORDER, MODE), 256, 0, ctx->stream>>>(a, plane, cells, dim, m, partials);
             rc = launch_status("wave_max");
             if (rc) return rc;
         }
@@ -575,7 +631,7 @@ struct GridState {
             int rc = choose_physics();
             if (rc) return rc;
         }
-        const int fused = fused_count(ORDER);
+        const int fused = fused_count(ORDER, MODE);
         if (!max_valid || last_bc != bc || std::memcmp(&last_params, &m, sizeof(m)) != 0 || n_partials != fused) {
             int rc = refresh_max(bc, m, fused);
             if (rc) return rc;

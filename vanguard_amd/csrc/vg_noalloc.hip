@@ -82,7 +82,6 @@ int launch_noalloc(hipStream_t s, double *base, double *cells, const double *wit
 {
     using P = EulerPhys;
     constexpr int NF = P::NF, G = (ORDER == 2) ? 2 : 1;
-    constexpr int BSX = vg::Tiles<P>::bsx, RX = vg::Tiles<P>::rx, BSY = vg::Tiles<P>::bsy, HY = vg::Tiles<P>::hy;
     const int gy = ny + 2 * G, gx = nx + 2 * G;
     const long long gcells = (long long)gy * gx;
     const long long plane = (gcells + 63) / 64 * 64;
@@ -108,13 +107,10 @@ int launch_noalloc(hipStream_t s, double *base, double *cells, const double *wit
     args.clk = clk;
     args.partials = nullptr;
     args.fixed_params = 1;
-    if (dir == 0) {
-        dim3 grid((gx + (BSX - 2 * G) - 1) / (BSX - 2 * G), (gy + RX - 1) / RX);
-        vg::sweep_x_kernel<P, ORDER, MODE, BSX, RX><<<grid, BSX, 0, s>>>(args);
-    } else {
-        dim3 grid((gx + BSY - 1) / BSY, (gy + HY - 1) / HY);
-        vg::sweep_y_kernel<P, ORDER, MODE, BSY, HY><<<grid, BSY, 0, s>>>(args);
-    }
+    const bool tiles = vg::small_tiles<P>(ORDER, MODE, gy, gx);
+    if (dir == 0) vg::launch_x<P, ORDER, MODE>(s, tiles, args);
+    else if (tiles) vg::launch_y_tile<P, ORDER, MODE, 256, 8>(s, args);
+    else vg::launch_y_walk<P, ORDER, MODE, vg::Tiles<P>::bsy, vg::Tiles<P>::hy>(s, args);
     const long long icells = (long long)ny * nx;
     interior_to_aos_kernel<NF><<<(int)std::min<long long>((icells + 255) / 256, 4096), 256, 0, s>>>(b, cells, plane, ny,
                                                                                                     nx, gx, G);

@@ -152,7 +152,7 @@ struct EulerPhys {
     // reference.
     __device__ static __forceinline__ void prim_to_cons_fast(const Params &m, const double (&w)[NF], double (&U)[NF])
     {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
         const double rho = w[0], u = w[1], v = w[2], z = w[3], p = w[4], lam = w[5];
         U[0] = rho;
         U[1] = rho * u;
@@ -163,15 +163,14 @@ struct EulerPhys {
     }
     __device__ static __forceinline__ void cons_to_prim_fast(const Params &m, const double (&U)[NF], double (&w)[NF])
     {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
         const double rho = U[0], r = rcp_nr(rho);
         const double u = U[1] * r, v = U[2] * r, z = U[3] * r, lam = U[5] * r;
-        const double ke = 0.5 * ((U[1] * u) + (U[2] * v) + (U[3] * z));
         w[0] = rho;
         w[1] = u;
         w[2] = v;
         w[3] = z;
-        w[4] = m.gm1 * (U[4] - ke - m.e_form * (U[5] - rho)) - m.gpinf;
+        w[4] = m.gm1 * (U[4] - 0.5 * (U[1] * u + U[2] * v + U[3] * z) - m.e_form * (U[5] - rho)) - m.gpinf;
         w[5] = lam;
     }
     // Flux from a primitive state and its conserved vector.
@@ -179,7 +178,7 @@ struct EulerPhys {
     __device__ static __forceinline__ void flux_prim_fast(const Params &m, const double (&w)[NF], const double (&U)[NF],
                                                           double (&F)[NF])
     {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
         (void)m;
         const double vn = (DIR == 0) ? w[1] : w[2];
         const double p = w[4];
@@ -287,7 +286,7 @@ struct EulerPlanarPhys {
     // FAST mode, as EulerPhys's.
     __device__ static __forceinline__ void prim_to_cons_fast(const Params &m, const double (&w)[NF], double (&U)[NF])
     {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
         const double rho = w[0], u = w[1], v = w[2], p = w[3];
         U[0] = rho;
         U[1] = rho * u;
@@ -296,20 +295,19 @@ struct EulerPlanarPhys {
     }
     __device__ static __forceinline__ void cons_to_prim_fast(const Params &m, const double (&U)[NF], double (&w)[NF])
     {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
         const double rho = U[0], r = rcp_nr(rho);
         const double u = U[1] * r, v = U[2] * r;
-        const double ke = 0.5 * ((U[1] * u) + (U[2] * v));
         w[0] = rho;
         w[1] = u;
         w[2] = v;
-        w[3] = m.gm1 * (U[3] - ke) - m.gpinf;
+        w[3] = m.gm1 * (U[3] - 0.5 * (U[1] * u + U[2] * v)) - m.gpinf;
     }
     template <int DIR>
     __device__ static __forceinline__ void flux_prim_fast(const Params &m, const double (&w)[NF], const double (&U)[NF],
                                                           double (&F)[NF])
     {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
         (void)m;
         const double vn = (DIR == 0) ? w[1] : w[2];
         const double p = w[3];

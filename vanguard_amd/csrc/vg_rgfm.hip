@@ -32,7 +32,6 @@ struct StepInternals {
 };
 
 struct RGFMGrid {
-    static constexpr int BSX = 256, RX = 4, BSY = 256, HY = 64;
     vg_ctx *ctx = nullptr;
     int dim = 2, ny = 1, nx = 1;
     long long cells = 0, plane = 0;
@@ -43,7 +42,7 @@ struct RGFMGrid {
     Clock *clk = nullptr, *tune_clk = nullptr;
     unsigned long long *partials = nullptr;
     int max_blocks = 0, circ_blocks = 0;
-    int y_variant = 0;                  // autotuned y-sweep shape
+    int y_variant = 0;                  // y-sweep shape (default_y, or autotuned)
     bool reduced = false;               // this run sweeps with the 4-field EulerPlanarPhys
     int *flag = nullptr;                // constant-plane check result
     hipGraphExec_t graph = nullptr;     // captured chunk of steps
@@ -58,6 +57,7 @@ struct RGFMGrid {
         nx = x;
         cells = (long long)ny * nx;
         plane = (cells + 63) / 64 * 64;
+        y_variant = default_y<EulerPhys>(2, VG_MODE_EXACT, ny, nx);
         for (int b = 0; b < 2; b++) {
             VG_HIP(hipMalloc(&m1[b], sizeof(double) * 6 * plane));
             VG_HIP(hipMalloc(&m2[b], sizeof(double) * 6 * plane));
@@ -176,10 +176,8 @@ struct RGFMGrid {
         a.clk = use_clk ? use_clk : clk;
         a.partials = nullptr;
         if (dir == 0) {
-            dim3 grid((nx + (BSX - 4) - 1) / (BSX - 4), (ny + RX - 1) / RX);
-            return ctx->timed("rgfm_sweep_x", [&] {
-                sweep_x_kernel<Q, 2, MODE, BSX, RX><<<grid, BSX, 0, ctx->stream>>>(a);
-            });
+            return ctx->timed("rgfm_sweep_x",
+                              [&] { launch_x<Q, 2, MODE>(ctx->stream, small_tiles<EulerPhys>(2, MODE, ny, nx), a); });
         }
         return launch_y<Q, 2, MODE>(ctx, y_variant, a);
     }

@@ -2,8 +2,9 @@
 // HPR) and the sweep direction, on register arrays.  EXACT mode follows the
 // reference's operation order (see the citations) with every product and sum
 // rounded separately; FAST mode is the same scheme with the primitive/conserved
-// round trips removed and multiply-adds fused (fp contract(fast) in its
-// branches only).
+// round trips removed and multiply-adds fused (fp contract(on) in its branches
+// only: a product is fused into the sum of its own expression, so every kernel
+// that inlines this code rounds alike, whatever its shape).
 #pragma once
 
 #include "vg_device.h"
@@ -69,7 +70,7 @@ __device__ __forceinline__ bool limiter_in_range(double num, double den)
 // FAST-mode limiter: the same piecewise functions with Newton-refined reciprocals.
 __device__ __forceinline__ double limiter_value_fast(double r, double bias, int limiter)
 {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
     if (r < 0.0) return 0.0;
     if (limiter == 0) {
         if (r < 0.5) return 2.0 * r;
@@ -183,7 +184,7 @@ struct Scheme {
                 xr[k] = xr[k] + evo;
             }
         } else {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
 #pragma unroll
             for (int k = 0; k < NF; k++) {
                 const double dl = UM[k] - UL[k];
@@ -200,9 +201,8 @@ struct Scheme {
             flux_of_cons(m, xr, Fr);
 #pragma unroll
             for (int k = 0; k < NF; k++) {
-                const double evo = half_c * (Fl[k] - Fr[k]);
-                xl[k] = xl[k] + evo;
-                xr[k] = xr[k] + evo;
+                xl[k] = xl[k] + half_c * (Fl[k] - Fr[k]);
+                xr[k] = xr[k] + half_c * (Fl[k] - Fr[k]);
             }
         }
         if (MODE == MODE_EXACT) {
@@ -253,7 +253,7 @@ struct Scheme {
 #pragma unroll
             for (int k = 0; k < NF; k++) F[k] = 0.5 * (lf[k] + ri[k]);
         } else {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
 #pragma unroll
             for (int k = 0; k < NF; k++) {
                 lf[k] = 0.5 * ((a.F[k] + b.F[k]) + (lf_c * (a.U[k] - b.U[k])));
@@ -276,7 +276,7 @@ struct Scheme {
             for (int k = 0; k < NF; k++) N[k] = U[k] + (up_c * (Fm[k] - Fp[k]));
             P::cons_to_prim(m, N, w);
         } else {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
 #pragma unroll
             for (int k = 0; k < NF; k++) N[k] = U[k] + (up_c * (Fm[k] - Fp[k]));
             P::cons_to_prim_fast(m, N, w);

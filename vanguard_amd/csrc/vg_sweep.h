@@ -82,21 +82,26 @@ __device__ __forceinline__ void block_max_to(unsigned long long *partials, unsig
     }
 }
 
-// One tile of an x sweep: thread tid holds the primitive state w of cell
-// j = j0 - G + tid (boundary-mapped by the caller); threads G .. BS-G-1 with
-// `write` set compute and store the updated cell at out[f * plane + out_idx].
-// Returns the wave-speed key of the stored cell when want_key (else 0).  Ends
-// with a barrier, so the LDS arrays can be reused by the next tile.
-template <class P, int ORDER, int MODE, int BS>
-__device__ __forceinline__ unsigned long long row_tile(const typename P::Params &m, const StepScalars &sc, double bias,
-                                                       int limiter, const double (&w)[P::NF], bool write,
-                                                       double *__restrict__ out, long long plane, long long out_idx,
-                                                       int dim, bool want_key, double *s_a, double *s_e)
+// One tile of a sweep along DIR: the block's threads are BS / LW positions along
+// the line by LW lines, thread tid holding position tid / LW of line tid % LW, so
+// its neighbours along the line are tid - LW and tid + LW (x tiles: LW = 1).
+// Thread tid holds the primitive state w of its cell, whose position in the grid
+// is the tile's first output - G + tid / LW (boundary-mapped by the caller);
+// positions G .. BS / LW - G - 1 with `write` set compute and store the updated
+// cell at out[f * plane + out_idx].  Returns the wave-speed key of the stored cell
+// when want_key (else 0).  Ends with a barrier, so the LDS arrays can be reused by
+// the next tile.
+template <class P, int DIR, int ORDER, int MODE, int BS, int LW>
+__device__ __forceinline__ unsigned long long line_tile(const typename P::Params &m, const StepScalars &sc, double bias,
+                                                        int limiter, const double (&w)[P::NF], bool write,
+                                                        double *__restrict__ out, long long plane, long long out_idx,
+                                                        int dim, bool want_key, double *s_a, double *s_e)
 {
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
-    using S = Scheme<P, 0, MODE>;
-    const int tid = threadIdx.x;
+    constexpr int NP = BS / LW;
+    using S = Scheme<P, DIR, MODE>;
+    const int tid = threadIdx.x, pos = tid / LW;
     double U[NF], Fp[NF];
     if (ORDER == 2) {
         S::cons(m, w, U);
@@ -104,12 +109,12 @@ __device__ __forceinline__ unsigned long long row_tile(const typename P::Params 
         for (int f = 0; f < NF; f++) s_a[f * BS + tid] = U[f];
         __syncthreads();
         ConsFlux<NF> left, right;
-        if (tid >= 1 && tid <= BS - 2) {
+        if (pos >= 1 && pos <= NP - 2) {
             double UL[NF], UR[NF];
 #pragma unroll
             for (int f = 0; f < NF; f++) {
-                UL[f] = s_a[f * BS + tid - 1];
-                UR[f] = s_a[f * BS + tid + 1];
+                UL[f] = s_a[f * BS + tid - LW];
+                UR[f] = s_a[f * BS + tid + LW];
             }
             S::evolve(m, UL, U, UR, bias, limiter, sc.half_c, left, right);
 #pragma unroll
@@ -119,14 +124,14 @@ __device__ __forceinline__ unsigned long long row_tile(const typename P::Params 
             }
         }
         __syncthreads();
-        if (tid >= 1 && tid <= BS - 3) {
+        if (pos >= 1 && pos <= NP - 3) {
             ConsFlux<NF> nb;
 #pragma unroll
             for (int f = 0; f < NF; f++) {
-                nb.U[f] = s_e[f * BS + tid + 1];
-                nb.F[f] = s_e[(NF + f) * BS + tid + 1];
+                nb.U[f] = s_e[f * BS + tid + LW];
+                nb.F[f] = s_e[(NF + f) * BS + tid + LW];
             }
-            S::force_face(m, right, nb, sc.lf_c, sc.ri_c, Fp);   // face j + 1/2
+            S::force_face(m, right, nb, sc.lf_c, sc.ri_c, Fp);   // face pos + 1/2
 #pragma unroll
             for (int f = 0; f < NF; f++) s_a[f * BS + tid] = Fp[f];
         }
@@ -141,12 +146,12 @@ __device__ __forceinline__ unsigned long long row_tile(const typename P::Params 
             s_e[(NF + f) * BS + tid] = cf.F[f];
         }
         __syncthreads();
-        if (tid <= BS - 2) {
+        if (pos <= NP - 2) {
             ConsFlux<NF> nb;
 #pragma unroll
             for (int f = 0; f < NF; f++) {
-                nb.U[f] = s_e[f * BS + tid + 1];
-                nb.F[f] = s_e[(NF + f) * BS + tid + 1];
+                nb.U[f] = s_e[f * BS + tid + LW];
+                nb.F[f] = s_e[(NF + f) * BS + tid + LW];
             }
             S::force_face(m, cf, nb, sc.lf_c, sc.ri_c, Fp);
 #pragma unroll
@@ -155,10 +160,10 @@ __device__ __forceinline__ unsigned long long row_tile(const typename P::Params 
         __syncthreads();
     }
     unsigned long long key = 0;
-    if (tid >= G && tid < BS - G && write) {
+    if (pos >= G && pos < NP - G && write) {
         double Fm[NF], wn[NF];
 #pragma unroll
-        for (int f = 0; f < NF; f++) Fm[f] = s_a[f * BS + tid - 1];
+        for (int f = 0; f < NF; f++) Fm[f] = s_a[f * BS + tid - LW];
         S::update(m, U, Fm, Fp, sc.up_c, wn);
         store_state<P>(out, plane, out_idx, wn);
         if (want_key) key = max_key(P::wave_speed(m, wn, dim));
@@ -200,11 +205,41 @@ __global__ __launch_bounds__(BS) void sweep_x_kernel(SweepArgs<P> a)
 #pragma unroll
         for (int f = 0; f < NF; f++) w[f] = wnext[f];
         if (i + 1 < i_end) load_state<P>(a.in, a.plane, row + nx + jj, wnext);
-        const unsigned long long k2 = row_tile<P, ORDER, MODE, BS>(m, sc, a.bias, a.limiter, w, j < nx, a.out, a.plane,
-                                                                   row + j, a.dim, a.fuse_max != 0, s_a, s_e);
+        const unsigned long long k2 = line_tile<P, 0, ORDER, MODE, BS, 1>(m, sc, a.bias, a.limiter, w, j < nx, a.out,
+                                                                          a.plane, row + j, a.dim, a.fuse_max != 0, s_a, s_e);
         key = (k2 > key) ? k2 : key;
     }
     if (a.fuse_max) block_max_to<BS>(a.partials, key);
+}
+
+// The y sweep in LDS tiles of LW columns by BS / LW rows, one cell per thread: the
+// whole sweep of a cell is one pass of the stencil instead of the walk below, at
+// the cost of the tile's halo rows (2 G of BS / LW) being computed twice.
+template <class P, int ORDER, int MODE, int BS, int LW>
+__global__ __launch_bounds__(BS) void sweep_y_tile_kernel(SweepArgs<P> a)
+{
+    constexpr int NF = P::NF;
+    constexpr int G = (ORDER == 2) ? 2 : 1;
+    constexpr int NP = BS / LW, OUT = NP - 2 * G;
+    __shared__ double s_a[NF * BS];
+    __shared__ double s_e[2 * NF * BS];
+
+    if (a.clk->done) return;
+    const double ts = a.clk->dt * a.dt_scale;
+    const StepScalars sc(ts, a.dx);
+    typename P::Params m = a.m;
+    if (ORDER == 2 && !a.fixed_params) P::begin_step(m, a.clk->S);   // first-order solvers never set c_h
+
+    const int tid = threadIdx.x;
+    const int ny = a.ny, nx = a.nx;
+    const int i = blockIdx.y * OUT - G + tid / LW, j = blockIdx.x * LW + tid % LW;
+    const int ii = (i >= -G && i < ny + G) ? ghost_index(i, ny, a.bc) : (i < 0 ? 0 : ny - 1);
+    const int jj = (j < nx) ? j : nx - 1;
+    double w[NF];
+    load_state<P>(a.in, a.plane, (long long)ii * nx + jj, w);
+    // The y sweep never ends a step, so it writes no CFL partials.
+    line_tile<P, 1, ORDER, MODE, BS, LW>(m, sc, a.bias, a.limiter, w, i < ny && j < nx, a.out, a.plane,
+                                         (long long)i * nx + j, a.dim, false, s_a, s_e);
 }
 
 // CPT columns per thread (j, j + BS, ...): their computations are independent,
@@ -348,7 +383,16 @@ __device__ __forceinline__ unsigned long long reduce_partials(const unsigned lon
 {
     __shared__ unsigned long long s_r[kReduceThreads / kWave];
     unsigned long long key = 0;
-    for (int k = threadIdx.x; k < n; k += kReduceThreads) key = (partials[k] > key) ? partials[k] : key;
+    // eight loads in flight: the small tiles of a 1531 x 1000 grid leave 26,027 slots
+    int k = threadIdx.x;
+    for (; k + 7 * kReduceThreads < n; k += 8 * kReduceThreads) {
+        unsigned long long v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = partials[k + q * kReduceThreads];
+#pragma unroll
+        for (int q = 0; q < 8; q++) key = (v[q] > key) ? v[q] : key;
+    }
+    for (; k < n; k += kReduceThreads) key = (partials[k] > key) ? partials[k] : key;
     key = wave_max_u64(key);
     if ((threadIdx.x & (kWave - 1)) == 0) s_r[threadIdx.x / kWave] = key;
     __syncthreads();
