@@ -288,7 +288,8 @@ typedef struct {
  * (mhdfirstordersolver.cpp:457-477) when order == 1, which neither sub-cycles
  * nor sets c_h (the c_h, c_p given here are its GLM constants).  Primitive
  * order (rho, u, v, w, p, Bx, By, Bz, psi), 9 doubles per cell.  Without
- * sub-cycles it runs as one persistent workgroup. */
+ * sub-cycles a short line runs as one persistent workgroup, a longer one as the
+ * 2D grids do. */
 int vg_mhd_solve_1d(vg_ctx *ctx, const double *prim_in, double *prim_out, int n, double dx, double cfl,
                     double t_final, int max_steps, double bias, int limiter, int order, int bc, int subcycles,
                     const vg_mhd_params *mp, int mode, double *dt_log, int dt_log_cap, vg_run_stats *stats);

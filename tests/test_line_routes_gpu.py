@@ -1,0 +1,88 @@
+"""1D solves by one workgroup and by the grid path, and the widths of the batch
+workgroup, at the sizes where the route or the width changes.  Add, multiply, divide
+and square root only: every comparison is bit for bit."""
+
+import math
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from vanguard_amd import _lib
+from vanguard_amd import solvers as S
+
+pytestmark = pytest.mark.gpu
+
+EULER = [1.4, 0, 25, 0, 0.25, 250]
+
+
+def _euler(n):
+    rng = np.random.default_rng(n)
+    w = rng.uniform(-0.4, 0.4, (n, 6))
+    w[:, 0], w[:, 4], w[:, 5] = rng.uniform(0.3, 1.5, n), rng.uniform(0.3, 1.5, n), 1.0
+    return w
+
+
+def _mhd(n, seed=0):
+    rng = np.random.default_rng(n + 100000 * seed)
+    w = rng.uniform(-0.4, 0.4, (n, 9))
+    w[:, 0], w[:, 4] = rng.uniform(0.5, 1.5, n), rng.uniform(0.5, 1.5, n)
+    return w
+
+
+# 252 / 253: one tile of 256 threads or of 512; 508 / 509 (SLIC) and 1020 / 1021
+# (FORCE): the last workgroup size and the first grid size; 60 / 124: MHD tiles.
+@pytest.mark.parametrize("n", [60, 124, 125, 252, 253, 508, 509, 569, 1020, 1021])
+@pytest.mark.parametrize("order", [2, 1])
+def test_1d_routes_match_oracle(vg_ctx, n, order):
+    kw = dict(order=order, dim=1, dx=1.0 / n, cfl=0.7, tfinal=math.inf, max_steps=11, bias=0.0, limiter=0)
+    for bc in (S.TRANSMISSIVE, S.PERIODIC):
+        w = _euler(n)
+        r = S.euler_solve(w, 1, 1.0 / n, 0.7, math.inf, order=order, limiter=0, max_steps=11, bc=bc)
+        ref, dts = O.euler_solve(w, params=EULER, bc=bc, **kw)
+        O.assert_bitwise(r.dt, dts, f"euler n {n} dt")
+        O.assert_bitwise(r.cells, ref, f"euler n {n} state")
+        w = _mhd(n)
+        r = S.mhd_solve(w, 1, 1.0 / n, 0.7, math.inf, order=order, limiter=0, max_steps=11, bc=bc,
+                        params=S.MHDMaterialParameters(5.0 / 3.0, 0.0, 0.7, 0.4))
+        ref, dts = O.mhd_solve(w, gamma=5.0 / 3.0, ch=0.7, cp=0.4, bc=bc, **kw)
+        O.assert_bitwise(r.dt, dts, f"mhd n {n} dt")
+        O.assert_bitwise(r.cells, ref, f"mhd n {n} state")
+
+
+@pytest.mark.parametrize("n", [300, 700])
+def test_final_time_and_caps_on_both_routes(vg_ctx, n):
+    w = _euler(n)
+    kw = dict(order=2, dim=1, dx=1.0 / n, cfl=0.8, bias=0.0, limiter=1, params=EULER)
+    ref, dts = O.euler_solve(w, tfinal=0.05, max_steps=0, **kw)
+    r = S.euler_solve(w, 1, 1.0 / n, 0.8, 0.05, limiter=1)
+    assert r.stats.t == 0.05 and r.stats.steps == len(dts)
+    O.assert_bitwise(r.dt, dts, "dt to the final time")
+    O.assert_bitwise(r.cells, ref, "state at the final time")
+    for cap in (1, 8, 9, 23):
+        r = S.euler_solve(w, 1, 1.0 / n, 0.8, 0.05, limiter=1, max_steps=cap)
+        assert r.stats.steps == cap
+        O.assert_bitwise(r.dt, dts[:cap], "capped dt prefix")
+    assert S.euler_solve(w, 1, 1.0 / n, 0.8, 0.0, limiter=1).stats.steps == 0
+
+
+@pytest.mark.parametrize("n", [300, 700])
+def test_a_step_that_cannot_advance_is_refused_on_both_routes(vg_ctx, n):
+    for solve, w, p in ((S.euler_solve, _euler(n), None), (S.mhd_solve, _mhd(n), S.MHDMaterialParameters(1.4))):
+        w[n // 2, 1] = math.inf          # an infinite wave speed: dt = 0
+        r = solve(w, 1, 1.0 / n, 0.8, 1.0, params=p, raise_on_error=False)
+        assert r.status == _lib.VG_ERR_NONFINITE and r.stats.steps == 0
+
+
+# 3 instances fill a wide workgroup each, 300 a middle one, 700 the narrow one.
+@pytest.mark.parametrize("n_inst", [3, 300, 700])
+@pytest.mark.parametrize("mode", [S.EXACT, S.FAST])
+def test_batch_widths_give_the_single_solves_bits(vg_ctx, n_inst, mode):
+    sizes = np.array([600, 300, 125] + [17 + (7 * q) % 120 for q in range(n_inst - 3)])
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    w = np.concatenate([_mhd(int(n), q) for q, n in enumerate(sizes)])
+    r = S.mhd_solve_batch(w, off, 1.0 / sizes, np.full(n_inst, 5.0 / 3.0), 10.0, 0.6, max_steps=7, limiter=1, mode=mode)
+    for q in (0, 1, 2, n_inst - 1):
+        one = S.mhd_solve(w[off[q]:off[q + 1]], 1, 1.0 / sizes[q], 0.6, 10.0, limiter=1, max_steps=7, mode=mode,
+                          params=S.MHDMaterialParameters(5.0 / 3.0))
+        O.assert_bitwise(r.cells[off[q]:off[q + 1]], one.cells, f"instance {q}")

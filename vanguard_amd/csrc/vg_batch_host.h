@@ -19,6 +19,7 @@
 #include <numeric>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "vg_batch.h"
@@ -42,35 +43,86 @@ struct BatchBuffers {
     }
 };
 
+// Workgroup widths of the batch kernel: the narrowest keeps the most instances
+// resident, the wider ones give an instance more of its CU where there are fewer
+// instances than that (MHD, 256 - 2048 cells, 192 instances: 65.4 us a step at 128
+// threads, 25.8 at 512; 500 instances: 85.8 at 128, 52.0 at 256).  The tile's 3 NF
+// doubles per thread in LDS end the widening; 1024 threads of an Euler tile took
+// 8.7 us a step against 5.4 for 512.
+template <class P>
+struct BatchWidths;
+
+// f(std::integral_constant<int, BS>) for the width bs.
+template <class P, class F>
+auto with_batch_width(int bs, const F &f)
+{
+    using W = BatchWidths<P>;
+    if (bs == W::wide) return f(std::integral_constant<int, W::wide>{});
+    if (bs == W::mid) return f(std::integral_constant<int, W::mid>{});
+    return f(std::integral_constant<int, W::narrow>{});
+}
+
+// f(std::integral_constant<int, ORDER>, std::integral_constant<int, MODE>)
+template <class F>
+auto with_order_mode(int order, int mode, const F &f)
+{
+    using std::integral_constant;
+    if (order == 2)
+        return mode == VG_MODE_EXACT ? f(integral_constant<int, 2>{}, integral_constant<int, 0>{})
+                                     : f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    return mode == VG_MODE_EXACT ? f(integral_constant<int, 1>{}, integral_constant<int, 0>{})
+                                 : f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+}
+
 // Workgroups of the batch kernel resident at once on the device.
-template <class P, int ORDER, int MODE, int BS>
-int batch_slots(vg_ctx *ctx)
+template <class P>
+int batch_slots(vg_ctx *ctx, int order, int mode, int bs)
 {
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batch_solve_kernel<P, ORDER, MODE, BS>, BS, 0) !=
-        hipSuccess)
-        per_cu = 1;
+    const hipError_t e = with_order_mode(order, mode, [&](auto o, auto md) {
+        return with_batch_width<P>(bs, [&](auto w) {
+            constexpr int BS = decltype(w)::value;
+            return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, batch_solve_kernel<P, decltype(o)::value, decltype(md)::value, BS>, BS, 0);
+        });
+    });
+    if (e != hipSuccess) per_cu = 1;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) cus = 1;
     return std::max(1, per_cu) * std::max(1, cus);
 }
 
-template <class P, int ORDER, int MODE, int BS>
-int launch_batch(vg_ctx *ctx, const BatchArgs<P> &args, int n_inst)
+// The width for n_inst instances of at most n_max cells: the narrowest whose tile
+// holds the largest instance, but none at which the instances no longer run all at
+// once.
+template <class P>
+int batch_width(vg_ctx *ctx, int order, int mode, int n_inst, long long n_max)
+{
+    using W = BatchWidths<P>;
+    const int G = (order == 2) ? 2 : 1;
+    int bs = W::narrow;
+    for (int wider : {W::mid, W::wide})
+        if (n_max > bs - 2 * G && batch_slots<P>(ctx, order, mode, wider) >= n_inst) bs = wider;
+    return bs;
+}
+
+template <class P>
+int launch_batch(vg_ctx *ctx, int order, int mode, int bs, const BatchArgs<P> &args, int n_inst)
 {
     return ctx->timed("batch_solve", [&] {
-        batch_solve_kernel<P, ORDER, MODE, BS><<<n_inst, BS, 0, ctx->stream>>>(args);
+        with_order_mode(order, mode, [&](auto o, auto md) {
+            with_batch_width<P>(bs, [&](auto w) {
+                constexpr int BS = decltype(w)::value;
+                batch_solve_kernel<P, decltype(o)::value, decltype(md)::value, BS>
+                    <<<n_inst, BS, 0, ctx->stream>>>(args);
+            });
+        });
     });
 }
 
-// prim_in / prim_out: all instances' cells, array of structures (NF doubles per cell).
-template <class P, int BS>
-int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offsets_h, const double *prim_in,
-              double *prim_out, const double *dx_h, const std::vector<typename P::Params> &params_h,
-              const double *t_final_h, double cfl, int max_steps, double bias, int limiter, int bc, double *dt_log_h,
-              int dt_cap, int32_t *steps_h, double *t_out_h, vg_run_stats *stats)
+inline int check_batch_args(int order, int mode, int n_inst, const int64_t *offsets_h, const double *prim_in,
+                            const double *prim_out, const double *dx_h, const double *t_final_h, double cfl,
+                            int max_steps, int bc)
 {
-    constexpr int NF = P::NF;
-    auto w0 = std::chrono::steady_clock::now();
     VG_CHECK(n_inst >= 1, "need at least one instance");
     VG_CHECK(offsets_h && prim_in && prim_out && dx_h && t_final_h, "null argument");
     VG_CHECK(order == 1 || order == 2, "order must be 1 (FORCE) or 2 (SLIC)");
@@ -85,7 +137,24 @@ int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offse
         VG_CHECK(dx_h[q] > 0.0 && std::isfinite(dx_h[q]), "cell spacing must be positive");
         VG_CHECK(max_steps > 0 || std::isfinite(t_final_h[q]), "an infinite final time needs a step cap");
     }
+    return VG_OK;
+}
+
+// prim_in / prim_out: all instances' cells, array of structures (NF doubles per cell).
+template <class P>
+int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offsets_h, const double *prim_in,
+              double *prim_out, const double *dx_h, const std::vector<typename P::Params> &params_h,
+              const double *t_final_h, double cfl, int max_steps, double bias, int limiter, int bc, double *dt_log_h,
+              int dt_cap, int32_t *steps_h, double *t_out_h, vg_run_stats *stats)
+{
+    constexpr int NF = P::NF;
+    auto w0 = std::chrono::steady_clock::now();
+    int rc = check_batch_args(order, mode, n_inst, offsets_h, prim_in, prim_out, dx_h, t_final_h, cfl, max_steps, bc);
+    if (rc) return rc;
     const long long cells = offsets_h[n_inst];
+    long long n_max = 0;
+    for (int q = 0; q < n_inst; q++) n_max = std::max<long long>(n_max, offsets_h[q + 1] - offsets_h[q]);
+    const int bs = batch_width<P>(ctx, order, mode, n_inst, n_max);
     BatchBuffers<P> b;
     VG_HIP(hipMalloc(&b.offsets, sizeof(long long) * (n_inst + 1)));
     VG_HIP(hipMalloc(&b.dx, sizeof(double) * n_inst));
@@ -110,7 +179,7 @@ int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offse
     VG_HIP(hipMemcpyAsync(b.staging, prim_in, sizeof(double) * NF * cells, hipMemcpyHostToDevice, s));
     const int gblocks = (int)std::min<long long>((cells + 255) / 256, 4096);
     batch_aos_to_planes<NF><<<gblocks, 256, 0, s>>>(b.staging, b.buf0, b.offsets, n_inst, cells);
-    int rc = launch_status("batch_aos_to_planes");
+    rc = launch_status("batch_aos_to_planes");
     if (rc) return rc;
 
     // Launch order: decreasing cells^2 * initial wave speed.
@@ -155,10 +224,7 @@ int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offse
     // time the others finish instead of holding it alone on one CU.
     double budget = 0.0;
     if (n_inst > 1) {
-        const int slots = (order == 2 && mode == 0)   ? batch_slots<P, 2, 0, BS>(ctx)
-                          : (order == 2)              ? batch_slots<P, 2, 1, BS>(ctx)
-                          : (mode == 0)               ? batch_slots<P, 1, 0, BS>(ctx)
-                                                      : batch_slots<P, 1, 1, BS>(ctx);
+        const int slots = batch_slots<P>(ctx, order, mode, bs);
         if (n_inst > slots) {
             std::vector<double> sp(n_inst);
             VG_HIP(hipMemcpyAsync(sp.data(), b.speed, sizeof(double) * n_inst, hipMemcpyDeviceToHost, s));
@@ -201,10 +267,7 @@ int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offse
     VG_HIP(hipEventCreate(&e0));
     VG_HIP(hipEventCreate(&e1));
     VG_HIP(hipEventRecord(e0, s));
-    if (order == 2 && mode == 0) rc = launch_batch<P, 2, 0, BS>(ctx, a, n_inst);
-    else if (order == 2) rc = launch_batch<P, 2, 1, BS>(ctx, a, n_inst);
-    else if (mode == 0) rc = launch_batch<P, 1, 0, BS>(ctx, a, n_inst);
-    else rc = launch_batch<P, 1, 1, BS>(ctx, a, n_inst);
+    rc = launch_batch<P>(ctx, order, mode, bs, a, n_inst);
     if (rc) return launch_status("batch_solve");
     VG_HIP(hipEventRecord(e1, s));
     batch_planes_to_aos<NF><<<gblocks, 256, 0, s>>>(b.buf0, b.buf1, b.where, b.staging, b.offsets, n_inst, cells);
@@ -339,6 +402,53 @@ int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offse
         return VG_ERR_NONFINITE;
     }
     return VG_OK;
+}
+
+// Cells up to which one 1D solve runs as a batch of one: a workgroup that holds
+// the grid in one tile (FORCE, half the work: two) needs no launch per step.  Beyond
+// it the grid path spreads the line over the device, its step length taken inside
+// the sweep (sweep_x_begin_kernel): one launch a step.  Microseconds a step,
+// workgroup / grid path, EXACT: Euler SLIC 500 cells 5.4 / 6.1, 750 cells 10.5 /
+// 6.2, 5000 cells 58 / 5.8 (256 threads); FORCE 500 cells 3.0 / 4.9, 1500 cells 9.8
+// / 5.0; MHD SLIC 500 cells 7.4 / 7.9, 5000 cells 154 / 8.1 (128 threads).
+template <class P>
+int one_workgroup_1d(int order)
+{
+    return order == 2 ? BatchWidths<P>::wide - 4 : 2 * (BatchWidths<P>::wide - 2);
+}
+
+// One whole 1D solve by the faster route.  scan: the grid path also fills the
+// stats' count of inadmissible cells.
+template <class P>
+int solve_line(vg_ctx *ctx, int order, int mode, const double *prim_in, double *prim_out, int n, double dx, double cfl,
+               double t_final, int max_steps, double bias, int limiter, int bc, const typename P::Params &m,
+               double *dt_log, int dt_cap, bool scan, vg_run_stats *stats)
+{
+    const int64_t offsets[2] = {0, n};
+    if (n <= one_workgroup_1d<P>(order)) {
+        std::vector<typename P::Params> params(1, m);
+        int32_t steps = 0;
+        double tend = 0.0;
+        const int rc = run_batch<P>(ctx, order, mode, 1, offsets, prim_in, prim_out, &dx, params, &t_final, cfl,
+                                    max_steps, bias, limiter, bc, dt_log, dt_cap, &steps, &tend, stats);
+        stats->steps = stats->total_steps = steps;
+        stats->t = tend;
+        return rc;
+    }
+    int rc = check_batch_args(order, mode, 1, offsets, prim_in, prim_out, &dx, &t_final, cfl, max_steps, bc);
+    if (rc) return rc;
+    GridState<P> g;
+    rc = g.create(ctx, 1, 1, n);
+    if (!rc) rc = g.load(prim_in, 0);
+    if (!rc) rc = g.run(order, mode, dx, cfl, t_final, max_steps, bias, limiter, bc, m, dt_log, dt_cap, stats);
+    if (!rc) rc = g.store(prim_out, 0);
+    if (!rc && g.stalled) {
+        set_error("1 instance(s) stopped because a time step could not advance t");
+        rc = VG_ERR_NONFINITE;
+    }
+    if (!rc && scan) rc = g.scan_nonfinite(m, &stats->nonfinite_cells, &stats->first_nonfinite);
+    g.destroy();
+    return rc;
 }
 
 }  // namespace vg

@@ -10,14 +10,16 @@
 
 using EulerGrid = vg::GridState<vg::EulerPhys>;
 
+template <>
+struct vg::BatchWidths<vg::EulerPhys> {
+    static constexpr int narrow = 256, mid = 512, wide = 512;
+};
+
 struct vg_euler_state {
     EulerGrid g;
 };
 
 namespace {
-
-// 1D grids up to this size run as one persistent workgroup.
-constexpr int kPersistent1D = 32768;
 
 vg::EulerPhys::Params to_params(const vg_euler_params *p)
 {
@@ -63,21 +65,13 @@ int solve(vg_ctx *ctx, int dim, const double *prim_in, double *prim_out, int ny,
     if (rc) return rc;
     rc = vg::bind(ctx);
     if (rc) return rc;
-    if (dim == 1 && nx <= kPersistent1D) {
-        // A small 1D grid runs its whole time loop in one persistent workgroup:
-        // one launch instead of a launch per step.
-        const int64_t offsets[2] = {0, nx};
-        std::vector<vg::EulerPhys::Params> params(1, to_params(mp));
-        int32_t steps = 0;
-        double tend = 0.0;
+    if (dim == 1) {
         vg_run_stats local{};
-        rc = vg::run_batch<vg::EulerPhys, 256>(ctx, order, mode, 1, offsets, prim_in, prim_out, &dx, params, &t_final,
-                                               cfl, max_steps, bias, limiter, bc, dt_log, dt_log_cap, &steps, &tend,
-                                               &local);
-        local.steps = local.total_steps = steps;
-        local.t = tend;
         local.first_nonfinite = -1;
-        for (int j = 0; j < nx && rc == VG_OK; j++) {
+        const bool one_workgroup = nx <= vg::one_workgroup_1d<vg::EulerPhys>(order);
+        rc = vg::solve_line<vg::EulerPhys>(ctx, order, mode, prim_in, prim_out, nx, dx, cfl, t_final, max_steps, bias,
+                                           limiter, bc, to_params(mp), dt_log, dt_log_cap, true, &local);
+        for (int j = 0; one_workgroup && j < nx && rc == VG_OK; j++) {
             const double *w = prim_out + 6 * (size_t)j;
             bool bad = !(w[0] > 0.0) || !((w[4] + mp->p_inf) > 0.0);
             for (int f = 0; f < 6; f++) bad = bad || !std::isfinite(w[f]);
@@ -273,7 +267,7 @@ extern "C" int vg_euler_solve_batch(vg_ctx *ctx, int n_inst, const int64_t *offs
     if (rc) return rc;
     std::vector<vg::EulerPhys::Params> params(n_inst);
     for (int q = 0; q < n_inst; q++) params[q] = to_params(&mp[q]);
-    return vg::run_batch<vg::EulerPhys, 256>(ctx, order, mode, n_inst, offsets, prim_in, prim_out, dx, params, t_final,
+    return vg::run_batch<vg::EulerPhys>(ctx, order, mode, n_inst, offsets, prim_in, prim_out, dx, params, t_final,
                                              cfl, max_steps, bias, limiter, VG_BC_TRANSMISSIVE, nullptr, 0, steps,
                                              t_out, stats);
 }

@@ -253,9 +253,12 @@ struct GridState {
     double *dt_dev = nullptr;      // device dt log (lazy)
     int dt_dev_cap = 0;
     unsigned long long *scan = nullptr;  // 2 counters for the non-finite scan
-    unsigned long long *partials = nullptr;  // per-block wave-speed keys
+    unsigned long long *partials = nullptr;  // per-block wave-speed keys (two sets, as the clock has two slots)
+    long long slots = 0;                     // keys per set
     int n_partials = 0;                      // slots written by the last producer
+    int tick = 0;                            // clock slot and key set of the step being enqueued (sweep_x_begin_kernel)
     bool max_valid = false;
+    bool stalled = false;          // the last run stopped on a step that could not advance t
     int subcycles = 0;             // source sub-cycles per half step (SourceStage)
     typename P::Params last_params{};
     int last_bc = -1;
@@ -280,14 +283,14 @@ struct GridState {
         plane = (cells + 63) / 64 * 64;
         VG_HIP(hipMalloc(&buf[0], sizeof(double) * NS * plane));
         VG_HIP(hipMalloc(&buf[1], sizeof(double) * NS * plane));
-        VG_HIP(hipMalloc(&clk, sizeof(Clock)));
+        VG_HIP(hipMalloc(&clk, 2 * sizeof(Clock)));
         VG_HIP(hipMalloc(&scan, 2 * sizeof(unsigned long long)));
         const long long gx = (nx + 64 - 4 - 1) / (64 - 4);
         // one per block of the largest producer: x sweep tiles of 64 cells, 64-cell
         // wave-speed blocks, or the source stage's tiles of 32 x 4 cells
         const long long tiles = (long long)((nx + 31) / 32) * ((ny + 3) / 4);
-        const long long slots = std::max<long long>(std::max<long long>(gx * ny, cells / 64 + 1), std::max(tiles, 4096LL));
-        VG_HIP(hipMalloc(&partials, sizeof(unsigned long long) * slots));
+        slots = std::max<long long>(std::max<long long>(gx * ny, cells / 64 + 1), std::max(tiles, 4096LL));
+        VG_HIP(hipMalloc(&partials, 2 * sizeof(unsigned long long) * slots));
         // stream-ordered copies only: a synchronous one would join the legacy
         // stream, which HIP refuses while another thread captures a graph
         Clock h{};
@@ -336,6 +339,7 @@ struct GridState {
         dt_dev_cap = o.dt_dev_cap;
         scan = o.scan;
         partials = o.partials;
+        slots = o.slots;
         n_partials = 0;
         max_valid = false;
         subcycles = o.subcycles;
@@ -441,7 +445,7 @@ struct GridState {
     template <class Q, int ORDER, int MODE>
     int launch_sweep_as(int dir, const double *in, double *out, double dt_scale, int fuse, int bc, double dx,
                         double bias, int limiter, const typename P::Params &m, Clock *use_clk = nullptr,
-                        int fixed_params = 0)
+                        int fixed_params = 0, const StepBegin *begin = nullptr)
     {
         SweepArgs<Q> a;
         a.in = in;
@@ -457,13 +461,16 @@ struct GridState {
         a.dim = dim;
         a.fuse_max = fuse;
         a.m = m;
-        a.clk = use_clk ? use_clk : clk;
-        a.partials = partials;
+        a.clk = use_clk ? use_clk : clk + tick;
+        a.partials = partials + tick * slots;
         a.fixed_params = fixed_params;
         if (dir == 0) {
             if (fuse) n_partials = fused_count(ORDER, MODE);
             return ctx->timed(ORDER == 2 ? "sweep_x_slic" : "sweep_x_force", [&] {
-                launch_x<Q, ORDER, MODE>(ctx->stream, small_tiles<P>(ORDER, MODE, ny, nx), a);
+                if (begin)
+                    sweep_x_begin_kernel<Q, ORDER, MODE><<<x_blocks<Q, ORDER>(true, ny, nx), kWave, 0, ctx->stream>>>(
+                        a, *begin);
+                else launch_x<Q, ORDER, MODE>(ctx->stream, small_tiles<P>(ORDER, MODE, ny, nx), a);
             });
         }
         // The y sweep never ends a step, so it never writes the CFL partials.
@@ -474,16 +481,16 @@ struct GridState {
     template <int ORDER, int MODE>
     int launch_sweep(int dir, const double *in, double *out, double dt_scale, int fuse, int bc, double dx,
                      double bias, int limiter, const typename P::Params &m, Clock *use_clk = nullptr,
-                     int fixed_params = 0)
+                     int fixed_params = 0, const StepBegin *begin = nullptr)
     {
         using R = typename ReducedPhys<P>::type;
         if constexpr (!std::is_void_v<R>) {
             if (reduced)
                 return launch_sweep_as<R, ORDER, MODE>(dir, in, out, dt_scale, fuse, bc, dx, bias, limiter, m, use_clk,
-                                                       fixed_params);
+                                                       fixed_params, begin);
         }
         return launch_sweep_as<P, ORDER, MODE>(dir, in, out, dt_scale, fuse, bc, dx, bias, limiter, m, use_clk,
-                                               fixed_params);
+                                               fixed_params, begin);
     }
 
     // One sweep of the current grid in direction dir with the caller's time step
@@ -554,26 +561,46 @@ struct GridState {
         return VG_OK;
     }
 
-    template <int ORDER, int MODE>
-    int enqueue_step(int bc, double dx, double bias, int limiter, const typename P::Params &m, double *dt_log, int dt_cap)
+    // Whether a captured step begins inside its first sweep (sweep_x_begin_kernel).
+    bool begins_in_sweep(int order, int mode, const typename P::Params &m) const
     {
-        clock_begin_kernel<<<1, kReduceThreads, 0, ctx->stream>>>(clk, partials, n_partials, dt_log, dt_cap);
-        int rc = launch_status("clock_begin");
+        if (order == 2 && ((SourceStage<P>::kActive && subcycles > 0) || PostStep<P>::active(m))) return false;
+        return n_partials <= kBeginSlots && small_tiles<P>(order, mode, ny, nx);
+    }
+
+    // One step.  `captured`: the step is recorded into a graph whose steps come in
+    // even numbers, so that the clock slots and key sets, of which a step that
+    // begins inside its first sweep uses one after the other, return to the first.
+    template <int ORDER, int MODE>
+    int enqueue_step(int bc, double dx, double bias, int limiter, const typename P::Params &m, double *dt_log, int dt_cap,
+                     bool captured = false)
+    {
+        const int nsub = (SourceStage<P>::kActive && ORDER == 2) ? subcycles : 0;
+        const bool post = ORDER == 2 && PostStep<P>::active(m);
+        StepBegin begin;
+        const bool fused_begin = captured && begins_in_sweep(ORDER, MODE, m);
+        int rc = VG_OK;
+        if (fused_begin) {
+            begin = StepBegin{clk + tick, clk + (1 - tick), partials + tick * slots, n_partials, dt_log, dt_cap};
+            tick = 1 - tick;
+        } else {
+            clock_begin_kernel<<<1, kReduceThreads, 0, ctx->stream>>>(clk, partials, n_partials, dt_log, dt_cap);
+            rc = launch_status("clock_begin");
+        }
         if (rc) return rc;
+        const StepBegin *bg = fused_begin ? &begin : nullptr;
         double *a = buf[cur], *b = buf[1 - cur];
         // Source half step before the sweeps (hprsecondordersolver.cpp:326-330, 514-520).
-        const int nsub = (SourceStage<P>::kActive && ORDER == 2) ? subcycles : 0;
         for (int s = 0; s < nsub; s++) {
             rc = SourceStage<P>::launch(*this, a, b, 0, bc, dx, bias, limiter, m);
             if (rc) return rc;
             std::swap(a, b);
         }
-        const bool post = ORDER == 2 && PostStep<P>::active(m);
         const int fuse = (nsub == 0 && !post) ? 1 : 0;
         if (dim == 1) {
-            rc = launch_sweep<ORDER, MODE>(0, a, b, 1.0, fuse, bc, dx, bias, limiter, m);
+            rc = launch_sweep<ORDER, MODE>(0, a, b, 1.0, fuse, bc, dx, bias, limiter, m, nullptr, 0, bg);
         } else {
-            rc = launch_sweep<ORDER, MODE>(0, a, b, 0.5, 0, bc, dx, bias, limiter, m);
+            rc = launch_sweep<ORDER, MODE>(0, a, b, 0.5, 0, bc, dx, bias, limiter, m, nullptr, 0, bg);
             if (!rc) rc = launch_sweep<ORDER, MODE>(1, b, a, 1.0, 0, bc, dx, bias, limiter, m);
             if (!rc) rc = launch_sweep<ORDER, MODE>(0, a, b, 0.5, fuse, bc, dx, bias, limiter, m);
         }
@@ -681,7 +708,21 @@ struct GridState {
         VG_HIP(hipEventCreate(&e1));
         VG_HIP(hipEventRecord(e0, ctx->stream));
         const int start_cur = cur;
-        const int chunk = (max_steps > 0 && max_steps <= 4096) ? max_steps : 256;
+        // Steps to enqueue before the clock is read again: what is left of the step
+        // cap, and of the way to the final time at the last step's length (before
+        // the start-up ramp is over, at the one its wave speed gives), so that few
+        // launches find the clock stopped.
+        auto steps_left = [&]() -> int {
+            const int most = (max_steps > 0 && max_steps <= 4096) ? 4096 : 256;
+            double left = most;
+            if (max_steps > 0) left = std::min(left, (double)max_steps - h.steps_this_run);
+            double S, dt = h.dt;
+            std::memcpy(&S, &h.smax, sizeof(S));
+            if (h.it <= 6) dt = cfl * (dx / std::max(S, h.corner));
+            const double e = (t_final - h.t) / dt + (h.it <= 6 ? 6.0 : 1.0);
+            if (e < left) left = e;   // false for a NaN
+            return std::max(1, (int)std::ceil(left));
+        };
         if (ctx->graphs && !ctx->timing) {
             // Capture kGraphSteps steps once (all kernels; no memory operations),
             // replay until the clock stops.  kGraphSteps is even, so every replay
@@ -701,10 +742,12 @@ struct GridState {
                 hipGraph_t g = nullptr;
                 VG_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
                 int rc = VG_OK;
-                for (int s = 0; s < kGraphSteps && !rc; s++) rc = enqueue_step<ORDER, MODE>(bc, dx, bias, limiter, m, dlog, dt_cap);
+                for (int s = 0; s < kGraphSteps && !rc; s++)
+                    rc = enqueue_step<ORDER, MODE>(bc, dx, bias, limiter, m, dlog, dt_cap, true);
                 hipError_t ec = hipStreamEndCapture(ctx->stream, &g);
                 if (rc) {
                     if (g) hipGraphDestroy(g);
+                    tick = 0;
                     return rc;
                 }
                 if (ec != hipSuccess) {
@@ -720,8 +763,8 @@ struct GridState {
                 }
                 graph_key = key;
             }
-            const int reps = std::max(1, chunk / kGraphSteps);
             for (;;) {
+                const int reps = (steps_left() + kGraphSteps - 1) / kGraphSteps;
                 for (int r = 0; r < reps; r++) VG_HIP(hipGraphLaunch(graph, ctx->stream));
                 VG_HIP(hipMemcpyAsync(&h, clk, sizeof(Clock), hipMemcpyDeviceToHost, ctx->stream));
                 VG_HIP(hipStreamSynchronize(ctx->stream));
@@ -730,6 +773,7 @@ struct GridState {
             }
         } else {
             for (;;) {
+                const int chunk = steps_left();
                 for (int s = 0; s < chunk; s++) {
                     int rc = enqueue_step<ORDER, MODE>(bc, dx, bias, limiter, m, dlog, dt_cap);
                     if (rc) return rc;
@@ -740,7 +784,8 @@ struct GridState {
                 if (max_steps > 0 && h.steps_this_run >= max_steps) break;
             }
         }
-        clock_finish_kernel<<<1, 1, 0, ctx->stream>>>(clk);
+        const bool two_sets = ctx->graphs && !ctx->timing && begins_in_sweep(ORDER, MODE, m);
+        clock_finish_kernel<<<1, 256, 0, ctx->stream>>>(clk, two_sets ? partials : nullptr, slots, n_partials);
         int rc = launch_status("clock_finish");
         if (rc) return rc;
         VG_HIP(hipEventRecord(e1, ctx->stream));
@@ -753,6 +798,7 @@ struct GridState {
         // Each executed step moved the grid to the other buffer; steps enqueued
         // after the loop condition failed did nothing.
         cur = start_cur ^ (h.steps_this_run & 1);
+        stalled = h.stalled != 0;
         if (dlog) {
             const int n = h.steps_this_run < dt_cap ? h.steps_this_run : dt_cap;
             if (n > 0) {

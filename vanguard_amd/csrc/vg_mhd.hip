@@ -7,14 +7,16 @@
 #include "vg_batch_host.h"
 #include "vg_mhd_host.h"
 
+template <>
+struct vg::BatchWidths<vg::MHDPhys> {
+    static constexpr int narrow = 128, mid = 256, wide = 512;
+};
+
 namespace {
 
 using vg::MHDPhys;
 
 MHDPhys::Params to_params(const vg_mhd_params *p) { return vg::mhd_params(p); }
-
-constexpr int kBatchBS = 128;
-
 
 // GridState path: 2D, or 1D with sub-cycles.
 int grid_solve(vg_ctx *ctx, int dim, const double *prim_in, double *prim_out, int ny, int nx, double dx, double cfl,
@@ -62,25 +64,16 @@ int vg_mhd_solve_1d(vg_ctx *ctx, const double *prim_in, double *prim_out, int n,
     VG_CHECK(mp != nullptr, "null material parameters");
     VG_CHECK(subcycles >= 0, "subcycles must be >= 0");
     if (order == 2 && subcycles > 0) {
-        // the source stage runs on the grid path; without it the one-instance
-        // persistent batch launch is the faster route
         VG_CHECK(n >= 2, "grid needs at least 2 cells");
         return grid_solve(ctx, 1, prim_in, prim_out, 1, n, dx, cfl, t_final, max_steps, bias, limiter, order, bc,
                           subcycles, mp, mode, dt_log, dt_log_cap, stats);
     }
     int rc = vg::bind(ctx);
     if (rc) return rc;
-    const int64_t offsets[2] = {0, n};
-    std::vector<MHDPhys::Params> params(1, to_params(mp));
-    int32_t steps = 0;
-    double tend = 0.0;
-    rc = vg::run_batch<MHDPhys, kBatchBS>(ctx, order, mode, 1, offsets, prim_in, prim_out, &dx, params, &t_final, cfl,
-                                          max_steps, bias, limiter, bc, dt_log, dt_log_cap, &steps, &tend, stats);
-    if (stats) {
-        stats->steps = steps;
-        stats->total_steps = steps;
-        stats->t = tend;
-    }
+    vg_run_stats local{};
+    rc = vg::solve_line<MHDPhys>(ctx, order, mode, prim_in, prim_out, n, dx, cfl, t_final, max_steps, bias, limiter, bc,
+                                 to_params(mp), dt_log, dt_log_cap, false, &local);
+    if (stats) *stats = local;
     return rc;
 }
 
@@ -105,9 +98,8 @@ int vg_mhd_solve_batch(vg_ctx *ctx, int n_inst, const int64_t *offsets, const do
     if (rc) return rc;
     std::vector<MHDPhys::Params> params(n_inst);
     for (int q = 0; q < n_inst; q++) params[q] = to_params(&mp[q]);
-    return vg::run_batch<MHDPhys, kBatchBS>(ctx, order, mode, n_inst, offsets, prim_in, prim_out, dx, params, t_final,
-                                            cfl, max_steps, bias, limiter, VG_BC_TRANSMISSIVE, nullptr, 0, steps,
-                                            t_out, stats);
+    return vg::run_batch<MHDPhys>(ctx, order, mode, n_inst, offsets, prim_in, prim_out, dx, params, t_final, cfl,
+                                  max_steps, bias, limiter, VG_BC_TRANSMISSIVE, nullptr, 0, steps, t_out, stats);
 }
 
 int vg_mhd_time_step_1d(vg_ctx *ctx, double *cells, const double *cells_with_boundary, int n, double dx, double dt,

@@ -172,8 +172,47 @@ __device__ __forceinline__ unsigned long long line_tile(const typename P::Params
     return key;
 }
 
+// Start of a step: finish the previous one (t += dt; it += 1 as in
+// secondordersolver.cpp:307-308), evaluate the loop condition, then
+// dt = CFL * (dx / S), x0.2 for the first six steps, clipped to the final time
+// (Solvers/solvers.cpp:392, 437-452).  mx: the wave-speed key of the grid.
+// Returns whether a step starts; the clock must not be done.
+__device__ __forceinline__ bool clock_advance(Clock &c, unsigned long long mx)
+{
+    c.smax = mx;
+    if (c.pending) {
+        c.t += c.dt;
+        c.it += 1;
+        c.pending = 0;
+    }
+    if (!(c.t < c.t_final) || (c.max_steps > 0 && c.it >= c.max_steps)) {
+        c.done = 1;
+        return false;
+    }
+    double S = __longlong_as_double((long long)mx);
+    if (c.corner > S) S = c.corner;
+    double dt = c.cfl * (c.dx / S);
+    if (c.it <= 5) dt *= 0.2;
+    if ((c.t + dt) > c.t_final) dt = c.t_final - c.t;
+    if (!(dt > 0.0) || !(c.t + dt > c.t)) {
+        // The reference would repeat this step forever (t never reaches t_final);
+        // stop and report instead.
+        c.done = 1;
+        c.stalled = 1;
+        return false;
+    }
+    c.dt = dt;
+    c.S = S;
+    if (c.steps_this_run == 0 || dt < c.dt_min) c.dt_min = dt;
+    if (c.steps_this_run == 0 || dt > c.dt_max) c.dt_max = dt;
+    c.steps_this_run += 1;
+    c.pending = 1;
+    return true;
+}
+
+// The rows of one x-sweep block, under time step dt and maximum wave speed S.
 template <class P, int ORDER, int MODE, int BS, int RX>
-__global__ __launch_bounds__(BS) void sweep_x_kernel(SweepArgs<P> a)
+__device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, double S)
 {
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
@@ -181,11 +220,10 @@ __global__ __launch_bounds__(BS) void sweep_x_kernel(SweepArgs<P> a)
     __shared__ double s_a[NF * BS];       // cell conserved vectors, later face fluxes
     __shared__ double s_e[2 * NF * BS];   // left evolved state (SLIC) / cell state (FORCE): U and F
 
-    if (a.clk->done) return;
-    const double ts = a.clk->dt * a.dt_scale;
+    const double ts = dt * a.dt_scale;
     const StepScalars sc(ts, a.dx);
     typename P::Params m = a.m;
-    if (ORDER == 2 && !a.fixed_params) P::begin_step(m, a.clk->S);   // first-order solvers never set c_h
+    if (ORDER == 2 && !a.fixed_params) P::begin_step(m, S);   // first-order solvers never set c_h
 
     const int tid = threadIdx.x;
     const int j = blockIdx.x * OUT - G + tid;
@@ -210,6 +248,52 @@ __global__ __launch_bounds__(BS) void sweep_x_kernel(SweepArgs<P> a)
         key = (k2 > key) ? k2 : key;
     }
     if (a.fuse_max) block_max_to<BS>(a.partials, key);
+}
+
+template <class P, int ORDER, int MODE, int BS, int RX>
+__global__ __launch_bounds__(BS) void sweep_x_kernel(SweepArgs<P> a)
+{
+    if (a.clk->done) return;
+    sweep_x_rows<P, ORDER, MODE, BS, RX>(a, a.clk->dt, a.clk->S);
+}
+
+// The first x sweep of a step together with the start of the step: every block
+// reduces the wave-speed keys of the last step and advances its own copy of the
+// clock, the first block writes the advanced clock and the dt log.  The advanced
+// clock is another slot than the one read (and the keys this sweep may write other
+// slots than those it reads), since blocks still to start read the old ones.
+// Bound by latency: of a 3.1 us clock_begin_kernel launch on a 200 x 200 grid 1.5
+// us remain here.  Every block reads every key, so it is for few keys only
+// (kBeginSlots).
+constexpr int kBeginSlots = 1024;
+
+struct StepBegin {
+    const Clock *from;
+    Clock *to;
+    const unsigned long long *keys;
+    int n_keys;
+    double *dt_log;
+    int dt_cap;
+};
+
+template <class P, int ORDER, int MODE>
+__global__ __launch_bounds__(kWave) void sweep_x_begin_kernel(SweepArgs<P> a, StepBegin b)
+{
+    Clock c = *b.from;
+    const bool first = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
+    bool run = false;
+    if (!c.done) {
+        unsigned long long key = 0;
+#pragma unroll 8
+        for (int k = threadIdx.x; k < b.n_keys; k += kWave) {
+            const unsigned long long v = b.keys[k];
+            key = (v > key) ? v : key;
+        }
+        run = clock_advance(c, wave_max_u64(key));
+        if (run && first && b.dt_log && c.steps_this_run <= b.dt_cap) b.dt_log[c.steps_this_run - 1] = c.dt;
+    }
+    if (first) *b.to = c;
+    if (run) sweep_x_rows<P, ORDER, MODE, kWave, 1>(a, c.dt, c.S);
 }
 
 // The y sweep in LDS tiles of LW columns by BS / LW rows, one cell per thread: the
@@ -418,51 +502,26 @@ __global__ void corner_speed_kernel(typename P::Params m, int dim, Clock *clk)
     clk->corner = P::wave_speed(m, w, dim);
 }
 
-// Start of a step: finish the previous one (t += dt; it += 1 as in
-// secondordersolver.cpp:307-308), evaluate the loop condition, then
-// dt = CFL * (dx / S), x0.2 for the first six steps, clipped to the final time
-// (Solvers/solvers.cpp:392, 437-452).
 static __global__ __launch_bounds__(kReduceThreads) void clock_begin_kernel(Clock *c, const unsigned long long *partials,
                                                                     int n_partials, double *dt_log, int dt_cap)
 {
     if (c->done) return;   // uniform: nothing pending once done
     const unsigned long long mx = reduce_partials(partials, n_partials);
     if (threadIdx.x != 0) return;
-    c->smax = mx;
-    if (c->pending) {
-        c->t += c->dt;
-        c->it += 1;
-        c->pending = 0;
-    }
-    if (c->done) return;
-    if (!(c->t < c->t_final) || (c->max_steps > 0 && c->it >= c->max_steps)) {
-        c->done = 1;
-        return;
-    }
-    double S = __longlong_as_double((long long)mx);
-    if (c->corner > S) S = c->corner;
-    double dt = c->cfl * (c->dx / S);
-    if (c->it <= 5) dt *= 0.2;
-    if ((c->t + dt) > c->t_final) dt = c->t_final - c->t;
-    if (!(dt > 0.0) || !(c->t + dt > c->t)) {
-        // The reference would repeat this step forever (t never reaches t_final);
-        // stop and report instead.
-        c->done = 1;
-        c->stalled = 1;
-        return;
-    }
-    c->dt = dt;
-    c->S = S;
-    if (dt_log && c->steps_this_run < dt_cap) dt_log[c->steps_this_run] = dt;
-    if (c->steps_this_run == 0 || dt < c->dt_min) c->dt_min = dt;
-    if (c->steps_this_run == 0 || dt > c->dt_max) c->dt_max = dt;
-    c->steps_this_run += 1;
-    c->pending = 1;
+    Clock h = *c;
+    if (clock_advance(h, mx) && dt_log && h.steps_this_run <= dt_cap) dt_log[h.steps_this_run - 1] = h.dt;
+    *c = h;
 }
 
-static __global__ void clock_finish_kernel(Clock *c)
+// End of a run: finishes its last step.  With `keys`, the run's steps began inside
+// their sweeps and left their wave-speed keys in two sets by turns: after an odd
+// number of steps the last keys, the second set's n, move to the first, where the
+// next run looks for them.
+static __global__ void clock_finish_kernel(Clock *c, unsigned long long *keys = nullptr, long long slots = 0, int n = 0)
 {
-    if (c->pending) {
+    if (keys && (c->steps_this_run & 1))
+        for (int k = threadIdx.x; k < n; k += blockDim.x) keys[k] = keys[slots + k];
+    if (threadIdx.x == 0 && c->pending) {
         c->t += c->dt;
         c->it += 1;
         c->pending = 0;
