@@ -496,6 +496,10 @@ int vg_rgfm_solve_fixed_dt_2d(vg_ctx *ctx, const double *m1_in, const double *m2
  * them in (vanguard_amd/csrc/vg_quot.h).  n <= 2^26. */
 int vg_division_selfcheck(vg_ctx *ctx, int64_t n, const double *a, const double *b, double *shared_q,
                           double *in_range_q, double *ieee_q);
+/* The same for the quotient by a scaled density, a / (c * b) (the specific internal
+ * energy's division by (gamma - 1) rho, whose reciprocal comes from rho's). */
+int vg_scaled_division_selfcheck(vg_ctx *ctx, int64_t n, const double *a, const double *b, const double *c,
+                                 double *scaled_q, double *ieee_q);
 
 /* ---- two-material ideal MHD: real ghost fluid method ------------------- */
 

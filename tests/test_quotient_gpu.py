@@ -133,3 +133,32 @@ def test_tiny_numerators():
     print(f"numerators below 2^-1000: {int((ulps > 0).sum())} of {deep.size} quotients differ, "
           f"at most {int(ulps.max())} ulp", flush=True)
     assert same_sign.all() and ulps.max() <= 1
+
+
+@pytest.mark.parametrize("scale", [0.4, 2.0 / 3.0, 0.648, 1.0, 6.12, 1.0 / 3.0, 2.0 ** -20 * 1.7, 2.0 ** 19 * 1.9])
+def test_quotients_by_a_scaled_density_are_ieee_division(scale):
+    """a / (c rho) with the reciprocal refined from rho's, c = gamma - 1: densities
+    2^-100 .. 2^100, scales 2^-20 .. 2^20, numerators as above; quotients next to
+    rounding midpoints and products c rho next to powers of two and all-ones
+    mantissas among them."""
+    rng = np.random.default_rng(105)
+    n = 1 << 21
+    a, rho = make(rng, n, -600, 599), make(rng, n, -100, 99, signed=False)
+    a[:64] = np.where(np.arange(64) % 2 == 0, 0.0, -0.0)
+    e, k = rng.integers(-70, 70, 20000), rng.integers(0, 64, 20000)
+    edge = np.ldexp(np.where(k % 2 == 0, 1.0 + k * 2.0 ** -52, 2.0 - k * 2.0 ** -52), e) / scale
+    m, b = near_midpoints(rng, 20000, e_b=(-60, 60))
+    rho = np.concatenate([rho, edge, b / scale])
+    a = np.concatenate([a, make(rng, 20000, -30, 30), m])
+    # midpoint numerators for the divisor the kernel forms
+    prod = scale * rho[-20000:]
+    a[-20000:] = [float((Fraction(q) + Fraction(np.spacing(abs(q))) / 2) * Fraction(float(p)))
+                  for q, p in zip(make(rng, 20000, -40, 40, signed=False), prod)]
+    ctx = S.default_context()
+    c = np.full(a.size, scale)
+    got, ieee = np.empty_like(a), np.empty_like(a)
+    rc = ctx.lib.vg_scaled_division_selfcheck(ctx.handle, a.size, *[_lib.as_dptr(np.ascontiguousarray(x))
+                                                                   for x in (a, rho, c)], _lib.as_dptr(got),
+                                              _lib.as_dptr(ieee))
+    assert rc == 0
+    assert_same(got, ieee, a, rho, f"scaled by {scale}")

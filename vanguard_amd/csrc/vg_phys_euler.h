@@ -54,6 +54,20 @@ struct EulerPhys {
         U[5] = rho * lam;
     }
 
+    // The same, given the shared divisor d of rho with d.fast, and scale_in_range(m.gm1).
+    __device__ static __forceinline__ void prim_to_cons_d(const Params &m, const double (&w)[NF],
+                                                          const SharedDivisor &d, double (&U)[NF])
+    {
+        const double rho = w[0], u = w[1], v = w[2], z = w[3], p = w[4], lam = w[5];
+        const double vsq = (u * u) + (v * v) + (z * z);
+        U[0] = rho;
+        U[1] = rho * u;
+        U[2] = rho * v;
+        U[3] = rho * z;
+        U[4] = rho * ((0.5 * vsq) + quot_scaled(p + m.gpinf, d, m.gm1, m.inv_gm1) + (m.e_form * (lam - 1.0)));
+        U[5] = rho * lam;
+    }
+
     // The quotients by rho of a conserved vector (u, v, w, lambda, E / rho), each
     // the correctly rounded IEEE quotient, from one shared reciprocal of rho.
     __device__ static __forceinline__ void by_rho(const double (&U)[NF], const SharedDivisor &d, double (&q)[5])
@@ -62,12 +76,12 @@ struct EulerPhys {
         quot_group<5>(a, d, q);
     }
 
-    // setConservedVariableVector (Euler/eulerstatevector.cpp:47-61); returns
-    // the shared divisor of rho for a flux of the same density.
-    __device__ static __forceinline__ SharedDivisor cons_to_prim_d(const Params &m, const double (&U)[NF], double (&w)[NF])
+    // setConservedVariableVector (Euler/eulerstatevector.cpp:47-61), given the
+    // shared divisor of rho.
+    __device__ static __forceinline__ void cons_to_prim_d(const Params &m, const double (&U)[NF],
+                                                          const SharedDivisor &d, double (&w)[NF])
     {
         const double rho = U[0];
-        const SharedDivisor d = shared_divisor(rho);
         double q[5];
         by_rho(U, d, q);
         const double u = q[0], v = q[1], z = q[2];
@@ -80,11 +94,10 @@ struct EulerPhys {
         w[3] = z;
         w[4] = eos_p(m, rho, e);
         w[5] = lam;
-        return d;
     }
     __device__ static __forceinline__ void cons_to_prim(const Params &m, const double (&U)[NF], double (&w)[NF])
     {
-        (void)cons_to_prim_d(m, U, w);
+        cons_to_prim_d(m, U, shared_divisor(U[0]), w);
     }
 
     // computeXFluxVector / computeYFluxVector of a conserved vector
@@ -216,15 +229,25 @@ struct EulerPlanarPhys {
         U[2] = rho * v;
         U[3] = rho * ((0.5 * vsq) + EulerPhys::eos_e(m, rho, p));
     }
+    __device__ static __forceinline__ void prim_to_cons_d(const Params &m, const double (&w)[NF],
+                                                          const SharedDivisor &d, double (&U)[NF])
+    {
+        const double rho = w[0], u = w[1], v = w[2], p = w[3];
+        const double vsq = (u * u) + (v * v);
+        U[0] = rho;
+        U[1] = rho * u;
+        U[2] = rho * v;
+        U[3] = rho * ((0.5 * vsq) + quot_scaled(p + m.gpinf, d, m.gm1, m.inv_gm1));
+    }
     __device__ static __forceinline__ void by_rho(const double (&U)[NF], const SharedDivisor &d, double (&q)[3])
     {
         const double a[3] = {U[1], U[2], U[3]};
         quot_group<3>(a, d, q);
     }
-    __device__ static __forceinline__ SharedDivisor cons_to_prim_d(const Params &m, const double (&U)[NF], double (&w)[NF])
+    __device__ static __forceinline__ void cons_to_prim_d(const Params &m, const double (&U)[NF],
+                                                          const SharedDivisor &d, double (&w)[NF])
     {
         const double rho = U[0];
-        const SharedDivisor d = shared_divisor(rho);
         double q[3];
         by_rho(U, d, q);
         const double u = q[0], v = q[1];
@@ -234,11 +257,10 @@ struct EulerPlanarPhys {
         w[1] = u;
         w[2] = v;
         w[3] = EulerPhys::eos_p(m, rho, e);
-        return d;
     }
     __device__ static __forceinline__ void cons_to_prim(const Params &m, const double (&U)[NF], double (&w)[NF])
     {
-        (void)cons_to_prim_d(m, U, w);
+        cons_to_prim_d(m, U, shared_divisor(U[0]), w);
     }
     template <int DIR>
     __device__ static __forceinline__ void flux_d(const Params &m, const double (&U)[NF], const SharedDivisor &d,

@@ -81,6 +81,25 @@ struct MHDPhys {
         U[8] = w[8];
     }
 
+    // The same, given the shared divisor d of rho with d.fast, and scale_in_range(m.gm1).
+    __device__ static __forceinline__ void prim_to_cons_d(const Params &m, const double (&w)[NF],
+                                                          const SharedDivisor &d, double (&U)[NF])
+    {
+        const double rho = w[0], u = w[1], v = w[2], z = w[3], p = w[4];
+        const double vsq = (u * u) + (v * v) + (z * z);
+        const double hydro = rho * ((0.5 * vsq) + quot_scaled(p + m.gpinf, d, m.gm1, m.inv_gm1));
+        const double b2 = (w[5] * w[5]) + (w[6] * w[6]) + (w[7] * w[7]);
+        U[0] = rho;
+        U[1] = rho * u;
+        U[2] = rho * v;
+        U[3] = rho * z;
+        U[4] = hydro + (0.5 * b2);
+        U[5] = w[5];
+        U[6] = w[6];
+        U[7] = w[7];
+        U[8] = w[8];
+    }
+
     // The quotients by rho of a conserved vector (u, v, w and the hydrodynamic
     // specific total energy (E - |B|^2 / 2) / rho), each the correctly rounded
     // IEEE quotient, from one shared reciprocal of rho.
@@ -91,13 +110,12 @@ struct MHDPhys {
         quot_group<4>(a, d, q);
     }
 
-    // setConservedVariableVector (mhdstatevector.cpp:49-68); returns the shared
-    // divisor of rho for a flux of the same density.
-    __device__ static __forceinline__ SharedDivisor cons_to_prim_d(const Params &m, const double (&U)[NF],
-                                                                   double (&w)[NF])
+    // setConservedVariableVector (mhdstatevector.cpp:49-68), given the shared
+    // divisor of rho.
+    __device__ static __forceinline__ void cons_to_prim_d(const Params &m, const double (&U)[NF],
+                                                          const SharedDivisor &d, double (&w)[NF])
     {
         const double rho = U[0];
-        const SharedDivisor d = shared_divisor(rho);
         const double bx = U[5], by = U[6], bz = U[7];
         const double b2 = (bx * bx) + (by * by) + (bz * bz);
         double q[4];
@@ -115,11 +133,10 @@ struct MHDPhys {
         w[6] = by;
         w[7] = bz;
         w[8] = U[8];
-        return d;
     }
     __device__ static __forceinline__ void cons_to_prim(const Params &m, const double (&U)[NF], double (&w)[NF])
     {
-        (void)cons_to_prim_d(m, U, w);
+        cons_to_prim_d(m, U, shared_divisor(U[0]), w);
     }
 
     // computeXFluxVector / computeYFluxVector (mhdstatevector.cpp:108-158,

@@ -126,6 +126,24 @@ VG_QUOT_FN double quot(double a, const SharedDivisor &d)
     return d.fast ? quot_refined(a, d) : a / d.b;
 }
 
+#ifdef __HIPCC__
+// RN(a / (c * d.b)) for a scale c with 2^-20 <= c <= 2^20 whose reciprocal is
+// c_inv, d.fast, and a in quot_refined's range: d's reciprocal times c_inv is within
+// two units of 1 / (c * d.b) in the last place, so one Newton step gives the
+// estimate that two give from the hardware's, and the quotient ends as it does
+// there.  Six instructions where the division sequence takes its own reciprocal.
+__device__ __forceinline__ double quot_scaled(double a, const SharedDivisor &d, double c, double c_inv)
+{
+    const double b = c * d.b;
+    double y = d.y * c_inv;
+    const double e = __builtin_fma(-b, y, 1.0);
+    y = __builtin_fma(y, e, y);
+    return div_finish(a, b, y);
+}
+// Whether c is a scale quot_scaled takes.
+__device__ __forceinline__ bool scale_in_range(double c) { return (c >= 0x1p-20) && (c <= 0x1p+20); }
+#endif
+
 // q[k] = RN(a[k] / d.b) for a group of numerators sharing the divisor: one
 // branch for the group, taken the same way by every lane of physical states.
 template <int N>

@@ -91,7 +91,7 @@ __device__ __forceinline__ void block_max_to(unsigned long long *partials, unsig
 // cell at out[f * plane + out_idx].  Returns the wave-speed key of the stored cell
 // when want_key (else 0).  Ends with a barrier, so the LDS arrays can be reused by
 // the next tile.
-template <class P, int DIR, int ORDER, int MODE, int BS, int LW>
+template <class P, int DIR, int ORDER, int MODE, int BS, int LW, bool FULL = false>
 __device__ __forceinline__ unsigned long long line_tile(const typename P::Params &m, const StepScalars &sc, double bias,
                                                         int limiter, const double (&w)[P::NF], bool write,
                                                         double *__restrict__ out, long long plane, long long out_idx,
@@ -100,7 +100,7 @@ __device__ __forceinline__ unsigned long long line_tile(const typename P::Params
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
     constexpr int NP = BS / LW;
-    using S = Scheme<P, DIR, MODE>;
+    using S = Scheme<P, DIR, MODE, FULL>;
     const int tid = threadIdx.x, pos = tid / LW;
     double U[NF], Fp[NF];
     if (ORDER == 2) {
@@ -243,8 +243,8 @@ __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, d
 #pragma unroll
         for (int f = 0; f < NF; f++) w[f] = wnext[f];
         if (i + 1 < i_end) load_state<P>(a.in, a.plane, row + nx + jj, wnext);
-        const unsigned long long k2 = line_tile<P, 0, ORDER, MODE, BS, 1>(m, sc, a.bias, a.limiter, w, j < nx, a.out,
-                                                                          a.plane, row + j, a.dim, a.fuse_max != 0, s_a, s_e);
+        const unsigned long long k2 = line_tile<P, 0, ORDER, MODE, BS, 1, (RX > 1)>(
+            m, sc, a.bias, a.limiter, w, j < nx, a.out, a.plane, row + j, a.dim, a.fuse_max != 0, s_a, s_e);
         key = (k2 > key) ? k2 : key;
     }
     if (a.fuse_max) block_max_to<BS>(a.partials, key);
@@ -326,16 +326,13 @@ __global__ __launch_bounds__(BS) void sweep_y_tile_kernel(SweepArgs<P> a)
                                          (long long)i * nx + j, a.dim, false, s_a, s_e);
 }
 
-// CPT columns per thread (j, j + BS, ...): their computations are independent,
-// so the instruction stream of a wave interleaves CPT dependency chains (the
-// divide sequences of EXACT mode are long chains); the arithmetic of every
-// cell is the same.  Columns past the grid's edge compute on the last column
-// and store nothing.
-template <class P, int ORDER, int MODE, int BS, int H, int CPT = 1>
+// A thread per column walks H rows with the stencil window in registers.  The y
+// sweep never ends a step, so it writes no CFL partials.
+template <class P, int ORDER, int MODE, int BS, int H>
 __global__ __launch_bounds__(BS) void sweep_y_kernel(SweepArgs<P> a)
 {
     constexpr int NF = P::NF;
-    using S = Scheme<P, 1, MODE>;
+    using S = Scheme<P, 1, MODE, true>;
 
     if (a.clk->done) return;
     const double ts = a.clk->dt * a.dt_scale;
@@ -343,103 +340,67 @@ __global__ __launch_bounds__(BS) void sweep_y_kernel(SweepArgs<P> a)
     typename P::Params m = a.m;
     if (ORDER == 2 && !a.fixed_params) P::begin_step(m, a.clk->S);   // first-order solvers never set c_h
 
-    const int j0 = blockIdx.x * BS * CPT + threadIdx.x;
+    const int j = blockIdx.x * BS + threadIdx.x;
     const int ny = a.ny, nx = a.nx;
     const int i0 = blockIdx.y * H;
     const int i1 = (i0 + H < ny) ? i0 + H : ny;
-    unsigned long long key = 0;
-
-    if (j0 < nx) {
-        int jc[CPT];
-        bool st[CPT];
+    if (j >= nx) return;
+    auto row_of = [&](int r) -> long long { return (long long)ghost_index(r, ny, a.bc) * nx + j; };
+    if (ORDER == 2) {
+        double A[NF], B[NF], C[NF], w[NF];
+        load_state<P>(a.in, a.plane, row_of(i0 - 2), w);
+        S::cons(m, w, A);
+        load_state<P>(a.in, a.plane, row_of(i0 - 1), w);
+        S::cons(m, w, B);
+        load_state<P>(a.in, a.plane, row_of(i0), w);   // row e + 1 of the first iteration
+        ConsFlux<NF> er_prev;
+        double Fprev[NF];
+        for (int e = i0 - 1; e <= i1; e++) {
+            S::cons(m, w, C);
+            if (e + 2 <= i1 + 1) load_state<P>(a.in, a.plane, row_of(e + 2), w);   // prefetch
+            ConsFlux<NF> L, R;
+            S::evolve(m, A, B, C, a.bias, a.limiter, sc.half_c, L, R);
+            double Fnew[NF];
+            if (e >= i0) S::force_face(m, er_prev, L, sc.lf_c, sc.ri_c, Fnew);   // face e - 1/2
+            if (e >= i0 + 1) {
+                double wn[NF];
+                S::update(m, A, Fprev, Fnew, sc.up_c, wn);                       // row e - 1
+                store_state<P>(a.out, a.plane, (long long)(e - 1) * nx + j, wn);
+            }
 #pragma unroll
-        for (int c = 0; c < CPT; c++) {
-            const int j = j0 + c * BS;
-            st[c] = j < nx;
-            jc[c] = st[c] ? j : nx - 1;
+            for (int f = 0; f < NF; f++) {
+                Fprev[f] = Fnew[f];
+                er_prev.U[f] = R.U[f];
+                er_prev.F[f] = R.F[f];
+                A[f] = B[f];
+                B[f] = C[f];
+            }
         }
-        auto row_of = [&](int r, int c) -> long long { return (long long)ghost_index(r, ny, a.bc) * nx + jc[c]; };
-        if (ORDER == 2) {
-            double A[CPT][NF], B[CPT][NF], C[CPT][NF], w[CPT][NF];
-#pragma unroll
-            for (int c = 0; c < CPT; c++) {
-                load_state<P>(a.in, a.plane, row_of(i0 - 2, c), w[c]);
-                S::cons(m, w[c], A[c]);
-                load_state<P>(a.in, a.plane, row_of(i0 - 1, c), w[c]);
-                S::cons(m, w[c], B[c]);
-                load_state<P>(a.in, a.plane, row_of(i0, c), w[c]);   // row e + 1 of the first iteration
+    } else {
+        double w[NF];
+        ConsFlux<NF> prev;
+        double Fprev[NF];
+        load_state<P>(a.in, a.plane, row_of(i0 - 1), w);
+        S::cons_flux_of_prim(m, w, prev);
+        for (int e = i0; e <= i1; e++) {
+            ConsFlux<NF> cur;
+            load_state<P>(a.in, a.plane, row_of(e), w);
+            S::cons_flux_of_prim(m, w, cur);
+            double Fnew[NF];
+            S::force_face(m, prev, cur, sc.lf_c, sc.ri_c, Fnew);                 // face e - 1/2
+            if (e >= i0 + 1) {
+                double wn[NF];
+                S::update(m, prev.U, Fprev, Fnew, sc.up_c, wn);                  // row e - 1
+                store_state<P>(a.out, a.plane, (long long)(e - 1) * nx + j, wn);
             }
-            ConsFlux<NF> er_prev[CPT];
-            double Fprev[CPT][NF];
-            for (int e = i0 - 1; e <= i1; e++) {
 #pragma unroll
-                for (int c = 0; c < CPT; c++) {
-                    S::cons(m, w[c], C[c]);
-                    if (e + 2 <= i1 + 1) load_state<P>(a.in, a.plane, row_of(e + 2, c), w[c]);   // prefetch
-                    ConsFlux<NF> L, R;
-                    S::evolve(m, A[c], B[c], C[c], a.bias, a.limiter, sc.half_c, L, R);
-                    double Fnew[NF];
-                    if (e >= i0) S::force_face(m, er_prev[c], L, sc.lf_c, sc.ri_c, Fnew);   // face e - 1/2
-                    if (e >= i0 + 1) {
-                        double wn[NF];
-                        S::update(m, A[c], Fprev[c], Fnew, sc.up_c, wn);                    // row e - 1
-                        if (st[c]) {
-                            store_state<P>(a.out, a.plane, (long long)(e - 1) * nx + jc[c], wn);
-                            if (a.fuse_max) {
-                                const unsigned long long k2 = max_key(P::wave_speed(m, wn, a.dim));
-                                key = (k2 > key) ? k2 : key;
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int f = 0; f < NF; f++) {
-                        Fprev[c][f] = Fnew[f];
-                        er_prev[c].U[f] = R.U[f];
-                        er_prev[c].F[f] = R.F[f];
-                        A[c][f] = B[c][f];
-                        B[c][f] = C[c][f];
-                    }
-                }
-            }
-        } else {
-            double w[CPT][NF];
-            ConsFlux<NF> prev[CPT];
-            double Fprev[CPT][NF];
-#pragma unroll
-            for (int c = 0; c < CPT; c++) {
-                load_state<P>(a.in, a.plane, row_of(i0 - 1, c), w[c]);
-                S::cons_flux_of_prim(m, w[c], prev[c]);
-            }
-            for (int e = i0; e <= i1; e++) {
-#pragma unroll
-                for (int c = 0; c < CPT; c++) {
-                    ConsFlux<NF> cur;
-                    load_state<P>(a.in, a.plane, row_of(e, c), w[c]);
-                    S::cons_flux_of_prim(m, w[c], cur);
-                    double Fnew[NF];
-                    S::force_face(m, prev[c], cur, sc.lf_c, sc.ri_c, Fnew);                 // face e - 1/2
-                    if (e >= i0 + 1) {
-                        double wn[NF];
-                        S::update(m, prev[c].U, Fprev[c], Fnew, sc.up_c, wn);               // row e - 1
-                        if (st[c]) {
-                            store_state<P>(a.out, a.plane, (long long)(e - 1) * nx + jc[c], wn);
-                            if (a.fuse_max) {
-                                const unsigned long long k2 = max_key(P::wave_speed(m, wn, a.dim));
-                                key = (k2 > key) ? k2 : key;
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int f = 0; f < NF; f++) {
-                        Fprev[c][f] = Fnew[f];
-                        prev[c].U[f] = cur.U[f];
-                        prev[c].F[f] = cur.F[f];
-                    }
-                }
+            for (int f = 0; f < NF; f++) {
+                Fprev[f] = Fnew[f];
+                prev.U[f] = cur.U[f];
+                prev.F[f] = cur.F[f];
             }
         }
     }
-    if (a.fuse_max) block_max_to<BS>(a.partials, key);
 }
 
 // Wave-speed maximum of a whole grid (the first step, or after the caller
