@@ -58,8 +58,14 @@ __device__ __forceinline__ unsigned long long block_allreduce_max(unsigned long 
     return mx;
 }
 
+// Waves per SIMD the batch kernel is compiled for: the nine-field state needs 176
+// registers, 8 over the limit for three waves, which large batches need to hide
+// their chains.
+template <class P, int BS>
+constexpr int kBatchWaves = (P::NF >= 9 && BS <= 256) ? 3 : 1;
+
 template <class P, int ORDER, int MODE, int BS>
-__global__ __launch_bounds__(BS) void batch_solve_kernel(BatchArgs<P> a)
+__global__ __launch_bounds__(BS, (kBatchWaves<P, BS>)) void batch_solve_kernel(BatchArgs<P> a)
 {
     constexpr int NF = P::NF;
     static_assert(StoredFields<P>::n == NF, "this kernel reads and writes all NF primitive planes");
@@ -124,7 +130,7 @@ __global__ __launch_bounds__(BS) void batch_solve_kernel(BatchArgs<P> a)
             double w[NF];
             load_prim<NF>(A, n, jj, w);
             const unsigned long long k2 =
-                line_tile<P, 0, ORDER, MODE, BS, 1>(m, sc, a.bias, a.limiter, w, j < n, B, n, j, 1, true, s_a, s_e);
+                line_tile<P, 0, ORDER, MODE, BS, 1, false, false>(m, sc, a.bias, a.limiter, w, j < n, B, n, j, 1, true, s_a, s_e);
             key = (k2 > key) ? k2 : key;
         }
         key = block_allreduce_max<BS>(key, s_red);   // its barriers also publish B for the next step

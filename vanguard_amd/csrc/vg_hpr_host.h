@@ -20,7 +20,7 @@ using HPRGrid = HPRGridT<0>;
 
 inline HPRParams hpr_to_params(const vg_hpr_params *p)
 {
-    HPRParams m;
+    HPRParams m{};
     m.is_thermal = p->is_thermal ? 1 : 0;
     m.is_plastic = p->is_plastic ? 1 : 0;
     m.rho0 = p->reference_density;
@@ -46,6 +46,9 @@ inline HPRParams hpr_to_params(const vg_hpr_params *p)
     m.cs2 = m.cs * m.cs;
     m.a2 = m.alpha * m.alpha;
     m.c02 = m.c0 * m.c0;
+    m.inv_G = 1.0 / m.G;
+    m.inv_Gcv = 1.0 / (m.G * m.cv);
+    m.short_div = scale_in_range(m.G) && scale_in_range(m.G * m.cv);
     return m;
 }
 

@@ -29,6 +29,10 @@ struct HPRParams {
     double G, cs2, a2;
     int eos;
     double p_ref, c0, gamma0, s_h, alpha_gr, sigma_y, n_pow, c02;
+    // reciprocals of G and G cv, estimates only (quot_near), and whether both are
+    // scales it takes
+    double inv_G, inv_Gcv;
+    int short_div;
 };
 
 // EOS: the equation of state, fixed per kernel (0 StiffenedGas, 1
@@ -142,6 +146,30 @@ struct HPRPhysT {
     }
     __device__ static __forceinline__ double mg_T_p(const Params &m, double rho) { return mg_e_p(m, rho) / m.cv; }
 
+    // The same, given the shared divisor d of rho: the stiffened gas divides by rho,
+    // rho Gamma and rho Gamma cv, whose reciprocals come from rho's where in range.
+    __device__ static __forceinline__ bool short_div(const Params &m, const SharedDivisor &d)
+    {
+        return EOS == 0 && d.fast && m.short_div;
+    }
+    __device__ static __forceinline__ double mg_e_d(const Params &m, double rho, double p, const SharedDivisor &d)
+    {
+        if (short_div(m, d))
+            return quot_refined(m.p_inf, d) + quot_near(p - mg_pref(m, rho), rho * m.G, d.y * m.inv_G);
+        return mg_e(m, rho, p);
+    }
+    __device__ static __forceinline__ double mg_p_d(const Params &m, double rho, double e, const SharedDivisor &d)
+    {
+        if (EOS == 0) return ((e - quot(m.p_inf, d)) * rho * m.G) + mg_pref(m, rho);
+        return mg_p(m, rho, e);
+    }
+    __device__ static __forceinline__ double mg_T_d(const Params &m, double rho, double p, const SharedDivisor &d)
+    {
+        if (short_div(m, d))
+            return m.t_ref + quot_near(p - mg_pref(m, rho), rho * m.G * m.cv, d.y * m.inv_Gcv);
+        return mg_T(m, rho, p);
+    }
+
     // ---- 3x3 helpers (Mathematics/matrixalgebra.cpp, tensoralgebra.cpp) ------------
     template <int NN>
     __device__ static __forceinline__ void load_A(const double (&s)[NN], double (&A)[3][3])
@@ -178,19 +206,32 @@ struct HPRPhysT {
                 c[i][j] = s;
             }
     }
-    // Gramian A^T A and its deviator G - (tr G / 3) I (tensoralgebra.cpp:22-30).
+    // Gramian A^T A and its deviator G - (tr G / 3) I (tensoralgebra.cpp:22-30), to
+    // the reference's bits with what cannot show left out: sums of squares are not
+    // begun at 0.0 (a square is never -0), the trace's third takes the short
+    // division, and off the diagonal, where the reference adds -1 * (third * 0.0) = -0,
+    // nothing is added (with an infinite or NaN trace the diagonal is NaN and every
+    // product of dev with it).
     __device__ static __forceinline__ void gram_dev(const double (&A)[3][3], double (&G)[3][3], double (&dev)[3][3])
     {
-        mul_tn(A, A, G);
-        double tr = 0.0;
-        tr = tr + G[0][0];
-        tr = tr + G[1][1];
-        tr = tr + G[2][2];
-        const double s = tr / 3.0;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            G[i][i] = (A[0][i] * A[0][i] + A[1][i] * A[1][i]) + A[2][i] * A[2][i];
+#pragma unroll
+            for (int j = i + 1; j < 3; j++) {
+                double s = 0.0;
+                s = s + A[0][i] * A[0][j];
+                s = s + A[1][i] * A[1][j];
+                s = s + A[2][i] * A[2][j];
+                G[i][j] = s;
+                G[j][i] = s;
+            }
+        }
+        const double s = third((G[0][0] + G[1][1]) + G[2][2]);
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 3; j++) dev[i][j] = G[i][j] + (-1.0 * (s * (i == j ? 1.0 : 0.0)));
+            for (int j = 0; j < 3; j++) dev[i][j] = (i == j) ? G[i][j] - s : G[i][j];
     }
     __device__ static __forceinline__ double det3(const double (&M)[3][3])
     {
@@ -203,16 +244,12 @@ struct HPRPhysT {
     {
         double G[3][3], dev[3][3];
         gram_dev(A, G, dev);
-        double total = 0.0;
+        // sums of squares, begun at their first term (never -0)
+        double row[3];
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-            double row = 0.0;
-            row = row + dev[i][0] * dev[i][0];
-            row = row + dev[i][1] * dev[i][1];
-            row = row + dev[i][2] * dev[i][2];
-            total = total + row;
-        }
-        return (0.25 * m.cs2) * total;
+        for (int i = 0; i < 3; i++)
+            row[i] = (dev[i][0] * dev[i][0] + dev[i][1] * dev[i][1]) + dev[i][2] * dev[i][2];
+        return (0.25 * m.cs2) * ((row[0] + row[1]) + row[2]);
     }
     __device__ static __forceinline__ double e_therm(const Params &m, double jx, double jy, double jz)
     {
@@ -223,11 +260,12 @@ struct HPRPhysT {
         return 0.5 * ((u * u) + (v * v) + (w * w));
     }
     __device__ static __forceinline__ double pressure_of(const Params &m, double rho, double E, double u, double v, double w,
-                                                         const double (&A)[3][3], double jx, double jy, double jz)
+                                                         const double (&A)[3][3], double jx, double jy, double jz,
+                                                         const SharedDivisor &d)
     {
         double e = E - (e_macro(u, v, w) + e_dist(m, A));
         if (m.is_thermal) e -= e_therm(m, jx, jy, jz);
-        return mg_p(m, rho, e);
+        return mg_p_d(m, rho, e, d);
     }
     // c_s^2 (A dev(A^T A)) (hprderivatives.cpp:17-24) and the shear stress
     // -rho A^T E_A with its density derivative -1 * A^T E_A (hprequationofstate.cpp:55-81).
@@ -254,10 +292,16 @@ struct HPRPhysT {
     // computeConservedVariableVector (hprstatevector.cpp:105-132).
     __device__ static __forceinline__ void prim_to_cons(const Params &m, const double (&w)[NF], double (&U)[NF])
     {
+        prim_to_cons_d(m, w, shared_divisor(w[0]), U);
+    }
+    // ... given the shared divisor of rho.
+    __device__ static __forceinline__ void prim_to_cons_d(const Params &m, const double (&w)[NF],
+                                                          const SharedDivisor &d, double (&U)[NF])
+    {
         double A[3][3];
         load_A(w, A);
         const double rho = w[0];
-        double E = mg_e(m, rho, w[1]) + e_dist(m, A) + e_macro(w[11], w[12], w[13]);
+        double E = mg_e_d(m, rho, w[1], d) + e_dist(m, A) + e_macro(w[11], w[12], w[13]);
         if (m.is_thermal) E += e_therm(m, w[14], w[15], w[16]);
         U[0] = rho;
         U[1] = rho * E;
@@ -279,20 +323,26 @@ struct HPRPhysT {
 
     // The quotients by rho of a conserved vector (u, v, w, J and E), each the
     // correctly rounded IEEE quotient, from one shared reciprocal of rho.
-    __device__ static __forceinline__ void by_rho(const double (&U)[NF], double (&q)[7])
+    __device__ static __forceinline__ void by_rho(const double (&U)[NF], const SharedDivisor &d, double (&q)[7])
     {
         const double a[7] = {U[11], U[12], U[13], U[14], U[15], U[16], U[1]};
-        quot_group<7>(a, shared_divisor(U[0]), q);
+        quot_group<7>(a, d, q);
     }
 
     // setConservedVariableVector (hprstatevector.cpp:59-76).
     __device__ static __forceinline__ void cons_to_prim(const Params &m, const double (&U)[NF], double (&w)[NF])
     {
+        cons_to_prim_d(m, U, shared_divisor(U[0]), w);
+    }
+    // ... given the shared divisor of rho.
+    __device__ static __forceinline__ void cons_to_prim_d(const Params &m, const double (&U)[NF],
+                                                          const SharedDivisor &d, double (&w)[NF])
+    {
         double A[3][3];
         load_A(U, A);
         const double rho = U[0];
         double q[7];
-        by_rho(U, q);
+        by_rho(U, d, q);
         const double u = q[0], v = q[1], z = q[2];
         double jx, jy, jz;
         if (m.is_thermal) {
@@ -306,7 +356,7 @@ struct HPRPhysT {
         }
         const double E = q[6];
         w[0] = rho;
-        w[1] = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz);
+        w[1] = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz, d);
 #pragma unroll
         for (int k = 2; k < 11; k++) w[k] = U[k];
         w[11] = u;
@@ -321,18 +371,25 @@ struct HPRPhysT {
     template <int DIR>
     __device__ static __forceinline__ void flux(const Params &m, const double (&U)[NF], double (&F)[NF])
     {
+        flux_of<DIR>(m, U, shared_divisor(U[0]), F);
+    }
+    // ... given the shared divisor of rho.
+    template <int DIR>
+    __device__ static __forceinline__ void flux_of(const Params &m, const double (&U)[NF], const SharedDivisor &d,
+                                                   double (&F)[NF])
+    {
         double A[3][3], sig[3][3], dsr[3][3];
         load_A(U, A);
         const double rho = U[0];
         shear(m, rho, A, sig, dsr);
         double q[7];
-        by_rho(U, q);
+        by_rho(U, d, q);
         const double u = q[0], v = q[1], z = q[2];
         const double jx = m.is_thermal ? q[3] : 0.0;
         const double jy = m.is_thermal ? q[4] : 0.0;
         const double jz = m.is_thermal ? q[5] : 0.0;
         const double E = q[6];
-        const double p = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz);
+        const double p = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz, d);
 #pragma unroll
         for (int k = 0; k < NF; k++) F[k] = 0.0;
         const double vn = (DIR == 0) ? u : v;
@@ -358,13 +415,26 @@ struct HPRPhysT {
             F[2 + 3 * i + DIR] = s;
         }
         if (m.is_thermal) {
-            const double T = mg_T(m, rho, p);
+            const double T = mg_T_d(m, rho, p, d);
             F[1] = F[1] + (T * (m.a2 * (DIR == 0 ? jx : jy)));
             F[14] = rho * (vn * jx);
             F[15] = rho * (vn * jy);
             F[16] = rho * (vn * jz);
             F[14 + DIR] = (rho * (vn * (DIR == 0 ? jx : jy))) + T;
         }
+    }
+
+    // setConservedVariableVector of x, then the conserved vector and flux of that
+    // state: rho comes back unchanged, so all three share its divisor.
+    template <int DIR>
+    __device__ static __forceinline__ void round_trip(const Params &m, const double (&x)[NF], double (&U)[NF],
+                                                      double (&F)[NF])
+    {
+        const SharedDivisor d = shared_divisor(x[0]);
+        double w[NF];
+        cons_to_prim_d(m, x, d, w);
+        prim_to_cons_d(m, w, d, U);
+        flux_of<DIR>(m, U, d, F);
     }
 
     // HPRAcousticTensor::computeMaximumWaveSpeed (hpracoustictensor.cpp:7-97) and
@@ -432,6 +502,7 @@ struct HPRPhysT {
                 M[i][j] = s;
             }
         double v[4] = {1.0, 1.0, 1.0, 1.0};
+#pragma clang loop unroll(disable)
         for (int it = 0; it < 10; it++) {
             double nv[4];
 #pragma unroll
@@ -522,11 +593,12 @@ struct HPRPhysT {
 #pragma unroll
             for (int j = 0; j < 3; j++) S[2 + 3 * i + j] = -(m.cs2 * Ad[i][j]) * th1;
         if (m.is_thermal) {
-            const double E = U[1] / rho;
-            const double u = U[11] / rho, v = U[12] / rho, z = U[13] / rho;
-            const double jx = U[14] / rho, jy = U[15] / rho, jz = U[16] / rho;
-            const double p = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz);
-            const double T = mg_T(m, rho, p);
+            const SharedDivisor d = shared_divisor(rho);
+            double q[7];
+            by_rho(U, d, q);
+            const double jx = q[3], jy = q[4], jz = q[5];
+            const double p = pressure_of(m, rho, q[6], q[0], q[1], q[2], A, jx, jy, jz, d);
+            const double T = mg_T_d(m, rho, p, d);
             const double th2 = 1.0 / (m.a2 * m.tau2 * ((rho / m.rho0) * (m.t0 / T)));
             S[14] = -rho * th2 * (m.a2 * jx);
             S[15] = -rho * th2 * (m.a2 * jy);

@@ -25,6 +25,18 @@ struct HasSharedDivisor<P, decltype((void)&P::template flux_d<0>)> {
     static constexpr bool value = true;
 };
 
+// Physics whose conversion to primitives, back, and flux share one divisor in a
+// function of their own (round_trip), a side at a time: two sides of the 17-field
+// state side by side would not fit the registers.
+template <class P, class = void>
+struct HasRoundTrip {
+    static constexpr bool value = false;
+};
+template <class P>
+struct HasRoundTrip<P, decltype((void)&P::template round_trip<0>)> {
+    static constexpr bool value = true;
+};
+
 // Correctly rounded division: the compiler's IEEE division, or the division
 // sequence without its scaling steps where the caller has shown the operands
 // in range (vg_quot.h).
@@ -60,15 +72,11 @@ __device__ __forceinline__ double limiter_value(double r, double bias, int limit
 // The limiter's divisions are in the range of the short division sequence when
 // every slope difference is at most 2^600 in magnitude (they are at least 1e-5
 // after the clamp) and -1 <= bias <= 1 (a NaN difference makes the limited slope NaN
-// by either division): then 2^-617 <= |r| <= 2^617, and the
-// denominators 1 + r and (1 - bias) + (1 + bias) r of the positive-r branches
-// lie in [2^-617, 2^619] with numerators 2 and 2r.
-__device__ __forceinline__ bool limiter_in_range(double num, double den)
-{
-    return smax(fabs(num), fabs(den)) <= 0x1p600;
-}
+// by either division): then 2^-617 <= |r| <= 2^617, and the denominators 1 + r and
+// (1 - bias) + (1 + bias) r of the positive-r branches lie in [2^-617, 2^619] with
+// numerators 2 and 2r.
 
-// d[k] *= limiter_value(num[k] / den[k]) for operands in range (limiter_in_range) and
+// d[k] *= limiter_value(num[k] / den[k]) for operands in that range and
 // -1 <= bias <= 1, every piece computed and the right one selected.
 template <int NF>
 __device__ __forceinline__ void limited_slopes(const double (&num)[NF], const double (&den)[NF], double bias, int limiter,
@@ -97,6 +105,108 @@ __device__ __forceinline__ void limited_slopes(const double (&num)[NF], const do
         for (int k = 0; k < NF; k++) {
             const double hi = fmin(1.0, R[k]);
             d[k] *= (r[k] < 0.0) ? 0.0 : ((r[k] < 1.0) ? r[k] : hi);
+        }
+    }
+}
+
+// limited_sides with IEEE divisions, for operands out of the short ones' range: no
+// state the solvers reach.  The fields are a loop over copies in scratch memory, so
+// that this path adds little code to the kernels of many fields.
+template <int NF, class NB>
+__device__ __forceinline__ void limited_sides_any_range(const NB &UL, const double (&UM)[NF], const NB &UR, double bias,
+                                                        int limiter, double (&xl)[NF], double (&xr)[NF])
+{
+    const double cl = 0.5 * (1.0 + bias), cr = 0.5 * (1.0 - bias);
+    double l[NF], c[NF], r[NF];
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+        l[k] = UL[k];
+        c[k] = UM[k];
+        r[k] = UR[k];
+    }
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < NF; k++) {
+        const double dl = c[k] - l[k];
+        const double dr = r[k] - c[k];
+        double d = (cl * dl) + (cr * dr);
+        const double num = (fabs(dl) < 1e-5) ? 1e-5 : dl;
+        const double den = (fabs(dr) < 1e-5) ? 1e-5 : dr;
+        d *= limiter_value(num / den, bias, limiter);
+        l[k] = c[k] - (0.5 * d);
+        r[k] = c[k] + (0.5 * d);
+    }
+#pragma unroll
+    for (int k = 0; k < NF; k++) {
+        xl[k] = l[k];
+        xr[k] = r[k];
+    }
+}
+
+// The middle cell's limited extrapolations to its two faces (EXACT).  Two cases need
+// no division: slope differences of opposite signs (r < 0, the limiters' zero piece)
+// and equal ones (r = 1 exactly, e.g. both clamped to 1e-5 in a flat region), whose
+// limiter value is the same for every cell.  GROUP > 0: that many fields at a time,
+// their division chains side by side (and no more slopes live at once); a wave all of
+// whose cells and fields are such cases takes them, any other every piece of every
+// field.  GROUP 0: branches, each lane taking its own pieces of a field at a time.
+template <int NF, int GROUP, class NB>
+__device__ __forceinline__ void limited_sides(const NB &UL, const double (&UM)[NF], const NB &UR, double bias, int limiter,
+                                              double (&xl)[NF], double (&xr)[NF])
+{
+    const double cl = 0.5 * (1.0 + bias), cr = 0.5 * (1.0 - bias);
+    double most = 0.0;
+#pragma unroll
+    for (int k = 0; k < NF; k++) most = fmax(fmax(most, fabs(UM[k] - UL[k])), fabs(UR[k] - UM[k]));
+    if (!(most <= 0x1p600 && (bias >= -1.0) && (bias <= 1.0))) {
+        limited_sides_any_range(UL, UM, UR, bias, limiter, xl, xr);
+        return;
+    }
+    const double f1 = limiter_value(1.0, bias, limiter, InRangeDiv());
+    if constexpr (GROUP == 0) {
+#pragma unroll
+        for (int k = 0; k < NF; k++) {
+            const double dl = UM[k] - UL[k];
+            const double dr = UR[k] - UM[k];
+            double d = (cl * dl) + (cr * dr);
+            const double num = (fabs(dl) < 1e-5) ? 1e-5 : dl;
+            const double den = (fabs(dr) < 1e-5) ? 1e-5 : dr;
+            double lim;
+            if (num * den < 0.0) lim = 0.0;
+            else if (num == den) lim = f1;
+            else lim = limiter_value(div_in_range(num, den), bias, limiter, InRangeDiv());
+            d *= lim;
+            xl[k] = UM[k] - (0.5 * d);
+            xr[k] = UM[k] + (0.5 * d);
+        }
+        return;
+    }
+    constexpr int N1 = GROUP > 0 ? GROUP : 1;
+#pragma unroll
+    for (int k0 = 0; k0 < NF; k0 += N1) {
+        double num[N1], den[N1], d[N1];
+        bool plain = true;
+#pragma unroll
+        for (int q = 0; q < N1; q++) {
+            const int k = (k0 + q < NF) ? k0 + q : NF - 1;
+            const double dl = UM[k] - UL[k];
+            const double dr = UR[k] - UM[k];
+            d[q] = (cl * dl) + (cr * dr);
+            // |difference| < 1e-5 is replaced by +1e-5 (sign dropped) before the ratio.
+            num[q] = (fabs(dl) < 1e-5) ? 1e-5 : dl;
+            den[q] = (fabs(dr) < 1e-5) ? 1e-5 : dr;
+            plain = plain && (num[q] * den[q] < 0.0 || num[q] == den[q]);
+        }
+        if (__all(plain)) {
+#pragma unroll
+            for (int q = 0; q < N1; q++) d[q] *= (num[q] == den[q]) ? f1 : 0.0;
+        } else {
+            limited_slopes(num, den, bias, limiter, d);
+        }
+#pragma unroll
+        for (int q = 0; q < N1; q++) {
+            if (k0 + q >= NF) continue;
+            xl[k0 + q] = UM[k0 + q] - (0.5 * d[q]);
+            xr[k0 + q] = UM[k0 + q] + (0.5 * d[q]);
         }
     }
 }
@@ -195,54 +305,7 @@ struct Scheme {
         double xl[NF], xr[NF];
         const double cl = 0.5 * (1.0 + bias), cr = 0.5 * (1.0 - bias);
         if constexpr (MODE == MODE_EXACT) {
-            double num[NF], den[NF], d[NF], most = 0.0;
-#pragma unroll
-            for (int k = 0; k < NF; k++) {
-                const double dl = UM[k] - UL[k];
-                const double dr = UR[k] - UM[k];
-                d[k] = (cl * dl) + (cr * dr);
-                // |difference| < 1e-5 is replaced by +1e-5 (sign dropped) before the ratio.
-                num[k] = (fabs(dl) < 1e-5) ? 1e-5 : dl;
-                den[k] = (fabs(dr) < 1e-5) ? 1e-5 : dr;
-                most = fmax(fmax(most, fabs(dl)), fabs(dr));
-            }
-            if (most <= 0x1p600 && (bias >= -1.0) && (bias <= 1.0)) {
-                // Two cases need no division: slope differences of opposite
-                // signs (r < 0, the limiters' zero piece) and equal ones (r = 1
-                // exactly, e.g. both clamped to 1e-5 in a flat region), whose
-                // limiter value is the same for every cell.
-                const double f1 = limiter_value(1.0, bias, limiter, InRangeDiv());
-                if constexpr (kLimiterBranches) {
-#pragma unroll
-                    for (int k = 0; k < NF; k++) {
-                        double lim;
-                        if (num[k] * den[k] < 0.0) lim = 0.0;
-                        else if (num[k] == den[k]) lim = f1;
-                        else lim = limiter_value(div_in_range(num[k], den[k]), bias, limiter, InRangeDiv());
-                        d[k] *= lim;
-                    }
-                } else {
-                    // a wave all of whose cells and fields are such cases, or all
-                    // pieces of every field
-                    bool plain = true;
-#pragma unroll
-                    for (int k = 0; k < NF; k++) plain = plain && (num[k] * den[k] < 0.0 || num[k] == den[k]);
-                    if (__all(plain)) {
-#pragma unroll
-                        for (int k = 0; k < NF; k++) d[k] *= (num[k] == den[k]) ? f1 : 0.0;
-                    } else {
-                        limited_slopes(num, den, bias, limiter, d);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < NF; k++) d[k] *= limiter_value(num[k] / den[k], bias, limiter);
-            }
-#pragma unroll
-            for (int k = 0; k < NF; k++) {
-                xl[k] = UM[k] - (0.5 * d[k]);
-                xr[k] = UM[k] + (0.5 * d[k]);
-            }
+            limited_sides<NF, kLimiterBranches ? 0 : (NF <= 9 ? NF : 3)>(UL, UM, UR, bias, limiter, xl, xr);
             double Fl[NF], Fr[NF];
             if constexpr (HasSharedDivisor<P>::value) {
                 // one branch for both sides, so their chains are scheduled together
@@ -304,6 +367,9 @@ struct Scheme {
                                   P::template flux_d<DIR>(m, left.U, sl, left.F);
                                   P::template flux_d<DIR>(m, right.U, sr, right.F);
                               });
+            } else if constexpr (HasRoundTrip<P>::value) {
+                P::template round_trip<DIR>(m, xl, left.U, left.F);
+                P::template round_trip<DIR>(m, xr, right.U, right.F);
             } else {
                 P::cons_to_prim(m, xl, w);
                 cons_flux_of_prim(m, w, left);

@@ -90,8 +90,10 @@ __device__ __forceinline__ void block_max_to(unsigned long long *partials, unsig
 // positions G .. BS / LW - G - 1 with `write` set compute and store the updated
 // cell at out[f * plane + out_idx].  Returns the wave-speed key of the stored cell
 // when want_key (else 0).  Ends with a barrier, so the LDS arrays can be reused by
-// the next tile.
-template <class P, int DIR, int ORDER, int MODE, int BS, int LW, bool FULL = false>
+// the next tile.  s_a and s_e hold NF and 2 NF fields per thread; COMPACT (SLIC): NF
+// and NF, the left evolved states taking s_a's place once the cells' vectors have been
+// read, at two more barriers for a third less LDS.
+template <class P, int DIR, int ORDER, int MODE, int BS, int LW, bool FULL, bool COMPACT>
 __device__ __forceinline__ unsigned long long line_tile(const typename P::Params &m, const StepScalars &sc, double bias,
                                                         int limiter, const double (&w)[P::NF], bool write,
                                                         double *__restrict__ out, long long plane, long long out_idx,
@@ -100,6 +102,7 @@ __device__ __forceinline__ unsigned long long line_tile(const typename P::Params
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
     constexpr int NP = BS / LW;
+    constexpr bool kCompact = COMPACT && ORDER == 2;
     using S = Scheme<P, DIR, MODE, FULL>;
     const int tid = threadIdx.x, pos = tid / LW;
     double U[NF], Fp[NF];
@@ -117,10 +120,14 @@ __device__ __forceinline__ unsigned long long line_tile(const typename P::Params
                 UR[f] = s_a[f * BS + tid + LW];
             }
             S::evolve(m, UL, U, UR, bias, limiter, sc.half_c, left, right);
+        }
+        double *s_u = kCompact ? s_a : s_e, *s_f = kCompact ? s_e : s_e + NF * BS;
+        if (kCompact) __syncthreads();   // every neighbour's vector has been read
+        if (pos >= 1 && pos <= NP - 2) {
 #pragma unroll
             for (int f = 0; f < NF; f++) {
-                s_e[f * BS + tid] = left.U[f];
-                s_e[(NF + f) * BS + tid] = left.F[f];
+                s_u[f * BS + tid] = left.U[f];
+                s_f[f * BS + tid] = left.F[f];
             }
         }
         __syncthreads();
@@ -128,10 +135,13 @@ __device__ __forceinline__ unsigned long long line_tile(const typename P::Params
             ConsFlux<NF> nb;
 #pragma unroll
             for (int f = 0; f < NF; f++) {
-                nb.U[f] = s_e[f * BS + tid + LW];
-                nb.F[f] = s_e[(NF + f) * BS + tid + LW];
+                nb.U[f] = s_u[f * BS + tid + LW];
+                nb.F[f] = s_f[f * BS + tid + LW];
             }
             S::force_face(m, right, nb, sc.lf_c, sc.ri_c, Fp);   // face pos + 1/2
+        }
+        if (kCompact) __syncthreads();   // every left state has been read
+        if (pos >= 1 && pos <= NP - 3) {
 #pragma unroll
             for (int f = 0; f < NF; f++) s_a[f * BS + tid] = Fp[f];
         }
@@ -210,6 +220,12 @@ __device__ __forceinline__ bool clock_advance(Clock &c, unsigned long long mx)
     return true;
 }
 
+// Whether the small tiles take the compact layout: where the block is one wave its
+// barriers cost nothing, and tiles of nine and more fields are bound by the waves
+// their LDS lets in (MHD y tiles 55 KB: two blocks of four waves a CU; 37 KB: four).
+template <class P, int ORDER, int BS>
+constexpr bool kCompactTile = ORDER == 2 && (P::NF >= 9 || BS == kWave);
+
 // The rows of one x-sweep block, under time step dt and maximum wave speed S.
 template <class P, int ORDER, int MODE, int BS, int RX>
 __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, double S)
@@ -217,8 +233,10 @@ __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, d
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
     constexpr int OUT = BS - 2 * G;
+    constexpr bool FULL = RX > 1, COMPACT = !FULL && kCompactTile<P, ORDER, BS>;
     __shared__ double s_a[NF * BS];       // cell conserved vectors, later face fluxes
-    __shared__ double s_e[2 * NF * BS];   // left evolved state (SLIC) / cell state (FORCE): U and F
+    // left evolved state (SLIC) / cell state (FORCE): U and F, or F only
+    __shared__ double s_e[(COMPACT ? 1 : 2) * NF * BS];
 
     const double ts = dt * a.dt_scale;
     const StepScalars sc(ts, a.dx);
@@ -230,22 +248,27 @@ __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, d
     const int nx = a.nx;
     const int jj = (j >= -G && j < nx + G) ? ghost_index(j, nx, a.bc) : (j < 0 ? 0 : nx - 1);
     const int i_begin = blockIdx.y * RX;
-    const int i_end = (i_begin + RX < a.ny) ? i_begin + RX : a.ny;
     unsigned long long key = 0;
-
-    // Each block walks RX rows; the next row's cells are loaded while the
-    // current row is computed.
+    auto tile = [&](int i, const double(&w)[NF]) {
+        const unsigned long long k2 = line_tile<P, 0, ORDER, MODE, BS, 1, FULL, COMPACT>(
+            m, sc, a.bias, a.limiter, w, j < nx, a.out, a.plane, (long long)i * nx + j, a.dim, a.fuse_max != 0, s_a, s_e);
+        key = (k2 > key) ? k2 : key;
+    };
     double wnext[NF];
     load_state<P>(a.in, a.plane, (long long)i_begin * nx + jj, wnext);
-    for (int i = i_begin; i < i_end; i++) {
-        const long long row = (long long)i * nx;
-        double w[NF];
+    if constexpr (RX == 1) {
+        tile(i_begin, wnext);
+    } else {
+        // Each block walks RX rows; the next row's cells are loaded while the
+        // current row is computed.
+        const int i_end = (i_begin + RX < a.ny) ? i_begin + RX : a.ny;
+        for (int i = i_begin; i < i_end; i++) {
+            double w[NF];
 #pragma unroll
-        for (int f = 0; f < NF; f++) w[f] = wnext[f];
-        if (i + 1 < i_end) load_state<P>(a.in, a.plane, row + nx + jj, wnext);
-        const unsigned long long k2 = line_tile<P, 0, ORDER, MODE, BS, 1, (RX > 1)>(
-            m, sc, a.bias, a.limiter, w, j < nx, a.out, a.plane, row + j, a.dim, a.fuse_max != 0, s_a, s_e);
-        key = (k2 > key) ? k2 : key;
+            for (int f = 0; f < NF; f++) w[f] = wnext[f];
+            if (i + 1 < i_end) load_state<P>(a.in, a.plane, (long long)(i + 1) * nx + jj, wnext);
+            tile(i, w);
+        }
     }
     if (a.fuse_max) block_max_to<BS>(a.partials, key);
 }
@@ -306,7 +329,8 @@ __global__ __launch_bounds__(BS) void sweep_y_tile_kernel(SweepArgs<P> a)
     constexpr int G = (ORDER == 2) ? 2 : 1;
     constexpr int NP = BS / LW, OUT = NP - 2 * G;
     __shared__ double s_a[NF * BS];
-    __shared__ double s_e[2 * NF * BS];
+    constexpr bool COMPACT = kCompactTile<P, ORDER, BS>;
+    __shared__ double s_e[(COMPACT ? 1 : 2) * NF * BS];
 
     if (a.clk->done) return;
     const double ts = a.clk->dt * a.dt_scale;
@@ -322,7 +346,7 @@ __global__ __launch_bounds__(BS) void sweep_y_tile_kernel(SweepArgs<P> a)
     double w[NF];
     load_state<P>(a.in, a.plane, (long long)ii * nx + jj, w);
     // The y sweep never ends a step, so it writes no CFL partials.
-    line_tile<P, 1, ORDER, MODE, BS, LW>(m, sc, a.bias, a.limiter, w, i < ny && j < nx, a.out, a.plane,
+    line_tile<P, 1, ORDER, MODE, BS, LW, false, COMPACT>(m, sc, a.bias, a.limiter, w, i < ny && j < nx, a.out, a.plane,
                                          (long long)i * nx + j, a.dim, false, s_a, s_e);
 }
 
