@@ -354,9 +354,19 @@ __device__ __forceinline__ void exact_interface(const State &a, const State &b, 
 
 // ---- line kernels -------------------------------------------------------------
 
-// Loop test of the step about to start (secondordersolver.cpp:295 style
-// `while (currentTime < finalTime)`): folds in the previous step and stops the
-// clock before anything of the next step runs.
+// Whether the loop test of the step about to start (secondordersolver.cpp:295 style
+// `while (currentTime < finalTime)`) fails, the previous step folded in: the kernels
+// that come before the step's clock_begin ask it themselves.
+__device__ __forceinline__ bool clock_stopped(const Clock *c)
+{
+    if (c->done) return true;
+    const double t = c->pending ? c->t + c->dt : c->t;
+    const int it = c->it + (c->pending ? 1 : 0);
+    return !(t < c->t_final) || (c->max_steps > 0 && it >= c->max_steps);
+}
+
+// The same test as a kernel that folds in the previous step and stops the clock
+// before anything of the next step runs.
 static __global__ void clock_check_kernel(Clock *c)
 {
     if (c->done) return;
@@ -398,6 +408,34 @@ __device__ __forceinline__ int block_exclusive_count(bool flag, int &total, int 
     return before + in_wave;
 }
 
+// The same for kLineBatch flags per thread, of positions tid, tid + kLineBS, ...: their
+// loads and ballots overlap, and one barrier pair serves them all.  s_w: kLineBatch
+// counts per wave.
+constexpr int kLineBatch = 4;
+
+__device__ __forceinline__ void block_exclusive_counts(const bool (&flag)[kLineBatch], int (&before)[kLineBatch],
+                                                       int &total, int *s_w)
+{
+    constexpr int W = kLineBS / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+#pragma unroll
+    for (int q = 0; q < kLineBatch; q++) {
+        const unsigned long long mask = __ballot(flag[q]);
+        before[q] = __popcll((lane == 0) ? 0ull : (mask & ((~0ull) >> (kWave - lane))));
+        if (lane == 0) s_w[q * W + wv] = __popcll(mask);
+    }
+    __syncthreads();
+    total = 0;
+#pragma unroll
+    for (int q = 0; q < kLineBatch; q++)
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+            if (k == wv) before[q] += total;
+            total += s_w[q * W + k];
+        }
+    __syncthreads();
+}
+
 struct LineArgs {
     double *m1, *m2;          // material planes (SoA, 6 fields), modified in place by the ghost fill
     const double *phi;        // level set
@@ -410,6 +448,7 @@ struct LineArgs {
     double h, dt_scale;       // level set: spacing along the line and fraction of dt
     EP p1, p2;
     const Clock *clk;
+    int test_stop = 0;        // ghost fill: runs before the step's clock_begin and asks clock_stopped
 };
 
 // Position k of line `line` -> flat cell index.
@@ -434,7 +473,7 @@ __global__ __launch_bounds__(kLineBS) void rgfm_fill_kernel(LineArgs a)
 {
     __shared__ unsigned char s_code[kMaxLine];   // 0: none; 1: crossing with flag 0; 2: with flag 1
     __shared__ int s_w[kLineBS / kWave];
-    if (a.clk->done) return;
+    if (a.test_stop ? clock_stopped(a.clk) : a.clk->done) return;
     const int line = blockIdx.x;
     const int n = (DIR == 0) ? a.nx : a.ny;
     const int tid = threadIdx.x;
@@ -509,6 +548,16 @@ __global__ __launch_bounds__(kLineBS) void rgfm_fill_kernel(LineArgs a)
     }
 }
 
+// phi at the middle of w (five neighbours along the line) after dt with velocity v:
+// the one-sided second-order upwind difference.
+__device__ __forceinline__ double level_set_update(const double (&w)[5], double v, double dt, double h)
+{
+    double up;
+    if (v < 0.0) up = (-w[4] + (4.0 * w[3]) - (3.0 * w[2])) / (2.0 * h);
+    else up = ((3.0 * w[2]) - (4.0 * w[1]) + w[0]) / (2.0 * h);
+    return w[2] - (dt * (v * up));
+}
+
 // updateLevelSetFunction / update2DLevelSetFunctionX/Y (rgfmsolver.cpp:493-646):
 // one workgroup per line; the material flag toggles at every sign change
 // (including position 0 against itself), the velocity component along the line
@@ -517,39 +566,37 @@ __global__ __launch_bounds__(kLineBS) void rgfm_fill_kernel(LineArgs a)
 template <int DIR>
 __global__ __launch_bounds__(kLineBS) void rgfm_level_set_kernel(LineArgs a)
 {
-    __shared__ int s_w[kLineBS / kWave];
+    __shared__ int s_w[kLineBatch * (kLineBS / kWave)];
     if (a.clk->done) return;
     const double dt = a.clk->dt * a.dt_scale;
     const int line = blockIdx.x;
     const int n = (DIR == 0) ? a.nx : a.ny;
     const int tid = threadIdx.x;
     int running = 0;
-    for (int k0 = 0; k0 < n; k0 += kLineBS) {
-        const int k = k0 + tid;
-        bool flag = false;
-        double c = 0.0;
-        if (k < n) {
-            c = a.phi[line_cell<DIR>(line, k, a.nx)];
-            const double pv = a.phi[line_cell<DIR>(line, k > 0 ? k - 1 : 0, a.nx)];
-            flag = (pv * c) <= 0.0;
-        }
-        int total;
-        const int before = block_exclusive_count(flag, total, s_w);
-        if (k < n) {
-            const int f = a.init_flag ^ ((running + before + (flag ? 1 : 0)) & 1);
-            const long long cell = line_cell<DIR>(line, k, a.nx);
-            const double v = (f ? a.m2 : a.m1)[(1 + DIR) * a.plane + cell];
-            double up;
-            if (v < 0.0) {
-                const double p2 = a.phi[line_cell<DIR>(line, ghost_index(k + 2, n, 0), a.nx)];
-                const double p1 = a.phi[line_cell<DIR>(line, ghost_index(k + 1, n, 0), a.nx)];
-                up = (-p2 + (4.0 * p1) - (3.0 * c)) / (2.0 * a.h);
-            } else {
-                const double m1v = a.phi[line_cell<DIR>(line, ghost_index(k - 1, n, 0), a.nx)];
-                const double m2v = a.phi[line_cell<DIR>(line, ghost_index(k - 2, n, 0), a.nx)];
-                up = ((3.0 * c) - (4.0 * m1v) + m2v) / (2.0 * a.h);
+    for (int k0 = 0; k0 < n; k0 += kLineBatch * kLineBS) {
+        // phi at k - 2 .. k + 2; the ghost at -1 is position 0, so the sign test of
+        // position 0 is against itself
+        double w[kLineBatch][5];
+        bool flag[kLineBatch];
+        int before[kLineBatch], total;
+#pragma unroll
+        for (int q = 0; q < kLineBatch; q++) {
+            const int k = k0 + q * kLineBS + tid;
+            flag[q] = false;
+            if (k < n) {
+#pragma unroll
+                for (int o = 0; o < 5; o++) w[q][o] = a.phi[line_cell<DIR>(line, ghost_index(k + o - 2, n, 0), a.nx)];
+                flag[q] = (w[q][1] * w[q][2]) <= 0.0;
             }
-            a.phi_out[cell] = c - (dt * (v * up));
+        }
+        block_exclusive_counts(flag, before, total, s_w);
+#pragma unroll
+        for (int q = 0; q < kLineBatch; q++) {
+            const int k = k0 + q * kLineBS + tid;
+            if (k >= n) continue;
+            const int f = a.init_flag ^ ((running + before[q] + (flag[q] ? 1 : 0)) & 1);
+            const long long cell = line_cell<DIR>(line, k, a.nx);
+            a.phi_out[cell] = level_set_update(w[q], (f ? a.m2 : a.m1)[(1 + DIR) * a.plane + cell], dt, a.h);
         }
         running += total;
     }
@@ -560,57 +607,75 @@ __global__ __launch_bounds__(kLineBS) void rgfm_level_set_kernel(LineArgs a)
 // rows, one thread per column segment, so each row read covers kLsCols
 // adjacent doubles (one workgroup per column, as in rgfm_level_set_kernel<1>,
 // reads one double per row at a stride of nx).  Pass 1 counts each segment's
-// sign changes; their prefix over the column's segments gives the count before
-// the segment; pass 2 walks the segment again, counting on, and updates phi.
-// The flag is that count's parity, so flags, velocities and the upwind
-// arithmetic are those of rgfm_level_set_kernel<1>, bit for bit.
-constexpr int kLsCols = 8, kLsSegs = 64;
+// sign changes; their prefix over the column's segments -- within a wave by shuffles,
+// over the waves' totals in LDS -- gives the count before the segment; pass 2 walks
+// the segment again, counting on, and updates phi, four rows at a time with their
+// loads in flight together.  The flag is that count's parity, so flags, velocities
+// and the upwind arithmetic are those of rgfm_level_set_kernel<1>, bit for bit.
+// Bound by latency (320 x 640: 11.3 us with a 64-step prefix in LDS and a row at a
+// time, 7.4 us so).
+constexpr int kLsCols = 8, kLsSegs = 64, kLsRows = 4;
 
 static __global__ __launch_bounds__(kLsCols * kLsSegs) void rgfm_level_set_y_kernel(LineArgs a)
 {
-    __shared__ int s_cnt[kLsSegs][kLsCols];
+    constexpr int W = kLsCols * kLsSegs / kWave;
+    __shared__ int s_tot[W][kLsCols];
     if (a.clk->done) return;
     const double dt = a.clk->dt * a.dt_scale;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
     const int cl = tid % kLsCols, seg = tid / kLsCols;
-    const int col = (int)blockIdx.x * kLsCols + cl;
     const int n = a.ny, nx = a.nx;
-    const bool ok = col < nx;
+    const bool ok = (int)blockIdx.x * kLsCols + cl < nx;
+    const int col = ok ? (int)blockIdx.x * kLsCols + cl : nx - 1;
     const int len = (n + kLsSegs - 1) / kLsSegs;
-    const int k0 = seg * len, k1 = (k0 + len < n) ? k0 + len : n;
+    const int k0 = (seg * len < n) ? seg * len : n, k1 = (k0 + len < n) ? k0 + len : n;
+    // phi of a position from -2 to n + 1 (later ones, which no row reads, as the last)
+    auto at = [&](int k) { return a.phi[(long long)ghost_index(k < n + 1 ? k : n + 1, n, 0) * nx + col]; };
     int cnt = 0;
-    if (ok) {
+    if (k0 < k1) {
+        double pv = at(k0 - 1);
 #pragma unroll 4
         for (int k = k0; k < k1; k++) {
             const double c = a.phi[(long long)k * nx + col];
-            const double pv = a.phi[(long long)(k > 0 ? k - 1 : 0) * nx + col];
             cnt += ((pv * c) <= 0.0) ? 1 : 0;
+            pv = c;
         }
     }
-    s_cnt[seg][cl] = cnt;
+    int run = cnt;
+#pragma unroll
+    for (int off = kLsCols; off < kWave; off <<= 1) {
+        const int o = __shfl_up(run, off, kWave);
+        if (lane >= off) run += o;
+    }
+    if (lane >= kWave - kLsCols) s_tot[wv][cl] = run;
+    run -= cnt;
     __syncthreads();
-    int run = 0;
-    for (int s2 = 0; s2 < seg; s2++) run += s_cnt[s2][cl];
+    for (int k = 0; k < wv; k++) run += s_tot[k][cl];
     if (!ok) return;
-#pragma unroll 4
-    for (int k = k0; k < k1; k++) {
-        const long long cell = (long long)k * nx + col;
-        const double c = a.phi[cell];
-        const double pv = a.phi[(long long)(k > 0 ? k - 1 : 0) * nx + col];
-        run += ((pv * c) <= 0.0) ? 1 : 0;
-        const int f = a.init_flag ^ (run & 1);
-        const double v = (f ? a.m2 : a.m1)[2 * a.plane + cell];
-        double up;
-        if (v < 0.0) {
-            const double p2 = a.phi[(long long)ghost_index(k + 2, n, 0) * nx + col];
-            const double p1 = a.phi[(long long)ghost_index(k + 1, n, 0) * nx + col];
-            up = (-p2 + (4.0 * p1) - (3.0 * c)) / (2.0 * a.h);
-        } else {
-            const double m1v = a.phi[(long long)ghost_index(k - 1, n, 0) * nx + col];
-            const double m2v = a.phi[(long long)ghost_index(k - 2, n, 0) * nx + col];
-            up = ((3.0 * c) - (4.0 * m1v) + m2v) / (2.0 * a.h);
+    double w[kLsRows + 4];
+    if (k0 < k1) {
+#pragma unroll
+        for (int o = 0; o < 4; o++) w[kLsRows + o] = at(k0 - 2 + o);
+    }
+    for (int kb = k0; kb < k1; kb += kLsRows) {
+#pragma unroll
+        for (int o = 0; o < 4; o++) w[o] = w[kLsRows + o];
+#pragma unroll
+        for (int o = 0; o < kLsRows; o++) w[4 + o] = at(kb + 2 + o);
+        double v[kLsRows];
+#pragma unroll
+        for (int r = 0; r < kLsRows; r++) {
+            run += ((w[r + 1] * w[r + 2]) <= 0.0) ? 1 : 0;   // a row past the segment's end counts for nobody
+            const int f = a.init_flag ^ (run & 1);
+            const int k = (kb + r < k1) ? kb + r : k1 - 1;
+            v[r] = (f ? a.m2 : a.m1)[2 * a.plane + (long long)k * nx + col];
         }
-        a.phi_out[cell] = c - (dt * (v * up));
+#pragma unroll
+        for (int r = 0; r < kLsRows; r++) {
+            if (kb + r >= k1) continue;
+            const double win[5] = {w[r], w[r + 1], w[r + 2], w[r + 3], w[r + 4]};
+            a.phi_out[(long long)(kb + r) * nx + col] = level_set_update(win, v[r], dt, a.h);
+        }
     }
 }
 

@@ -323,7 +323,7 @@ __global__ __launch_bounds__(kWave) void sweep_x_begin_kernel(SweepArgs<P> a, St
 // whole sweep of a cell is one pass of the stencil instead of the walk below, at
 // the cost of the tile's halo rows (2 G of BS / LW) being computed twice.
 template <class P, int ORDER, int MODE, int BS, int LW>
-__global__ __launch_bounds__(BS) void sweep_y_tile_kernel(SweepArgs<P> a)
+__device__ __forceinline__ void sweep_y_tile(const SweepArgs<P> &a)
 {
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
@@ -348,6 +348,35 @@ __global__ __launch_bounds__(BS) void sweep_y_tile_kernel(SweepArgs<P> a)
     // The y sweep never ends a step, so it writes no CFL partials.
     line_tile<P, 1, ORDER, MODE, BS, LW, false, COMPACT>(m, sc, a.bias, a.limiter, w, i < ny && j < nx, a.out, a.plane,
                                          (long long)i * nx + j, a.dim, false, s_a, s_e);
+}
+
+template <class P, int ORDER, int MODE, int BS, int LW>
+__global__ __launch_bounds__(BS) void sweep_y_tile_kernel(SweepArgs<P> a)
+{
+    sweep_y_tile<P, ORDER, MODE, BS, LW>(a);
+}
+
+// The tile sweeps of two grids of one shape in one launch (the launch's third
+// dimension picks the grid): on small grids one grid's tiles leave the device half
+// empty.
+template <class P>
+struct SweepPair {
+    SweepArgs<P> a, b;
+};
+
+template <class P, int ORDER, int MODE>
+__global__ __launch_bounds__(kWave) void sweep_x_pair_kernel(SweepPair<P> p)
+{
+    const SweepArgs<P> a = blockIdx.z ? p.b : p.a;
+    if (a.clk->done) return;
+    sweep_x_rows<P, ORDER, MODE, kWave, 1>(a, a.clk->dt, a.clk->S);
+}
+
+template <class P, int ORDER, int MODE, int BS, int LW>
+__global__ __launch_bounds__(BS) void sweep_y_tile_pair_kernel(SweepPair<P> p)
+{
+    const SweepArgs<P> a = blockIdx.z ? p.b : p.a;
+    sweep_y_tile<P, ORDER, MODE, BS, LW>(a);
 }
 
 // A thread per column walks H rows with the stencil window in registers.  The y
@@ -434,6 +463,26 @@ __global__ __launch_bounds__(256) void wave_max_kernel(const double *__restrict_
                                                        int dim, typename P::Params m, unsigned long long *partials)
 {
     constexpr int NF = P::NF;
+    unsigned long long key = 0;
+    for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < cells; c += (long long)gridDim.x * blockDim.x) {
+        double w[NF];
+        load_prim<NF>(in, plane, c, w);
+        const unsigned long long k2 = max_key(P::wave_speed(m, w, dim));
+        key = (k2 > key) ? k2 : key;
+    }
+    block_max_to<256>(partials, key);
+}
+
+// The same of two grids, the second's keys after the first's.
+template <class P>
+__global__ __launch_bounds__(256) void wave_max_pair_kernel(const double *__restrict__ in_a, const double *__restrict__ in_b,
+                                                            long long plane, long long cells, int dim,
+                                                            typename P::Params ma, typename P::Params mb,
+                                                            unsigned long long *partials)
+{
+    constexpr int NF = P::NF;
+    const double *in = blockIdx.y ? in_b : in_a;
+    const typename P::Params m = blockIdx.y ? mb : ma;
     unsigned long long key = 0;
     for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < cells; c += (long long)gridDim.x * blockDim.x) {
         double w[NF];
