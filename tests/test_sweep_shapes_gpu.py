@@ -69,7 +69,7 @@ def test_tile_edges_match_oracle(vg_ctx, physics, ny, nx):
 @pytest.mark.parametrize("physics,ny,nx,rep", [("euler", 133, 134, 10), ("mhd", 109, 110, 10), ("hpr", 82, 83, 10)])
 def test_large_grids_take_the_walking_sweeps_with_the_same_bits(vg_ctx, physics, ny, nx, rep):
     """A periodic state repeated over a grid beyond the small-tile rule (over 160 MB
-    read and written per sweep; FORCE 96 MB) advances as its repeated unit does: the walking
+    read and written per sweep; FORCE 48 MB) advances as its repeated unit does: the walking
     sweeps against the tiles."""
     unit = _state(physics, ny, nx)
     big = np.ascontiguousarray(np.tile(unit, (rep, rep, 1)))

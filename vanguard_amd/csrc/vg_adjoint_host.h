@@ -85,12 +85,9 @@ inline int adj_sweep(vg_ctx *ctx, int dir, int variant, const double *w, const d
     const int lines = (dir == 0) ? ny : nx;
     return ctx->timed(dir == 0 ? "adjoint_sweep_x" : "adjoint_sweep_y", [&] {
         launch_adjoint_dir<A>(ctx, dir, variant, a);
-        if (dir == 0)
-            euler_adjoint_fold_kernel<A, 0><<<(lines + 255) / 256, 256, 0, ctx->stream>>>(wbar_in, ghost, plane, ny,
-                                                                                               nx, bc);
-        else
-            euler_adjoint_fold_kernel<A, 1><<<(lines + 255) / 256, 256, 0, ctx->stream>>>(wbar_in, ghost, plane, ny,
-                                                                                               nx, bc);
+        const dim3 grid((lines + kWave - 1) / kWave, A::NF);
+        if (dir == 0) euler_adjoint_fold_kernel<A, 0><<<grid, kWave, 0, ctx->stream>>>(wbar_in, ghost, plane, ny, nx, bc);
+        else euler_adjoint_fold_kernel<A, 1><<<grid, kWave, 0, ctx->stream>>>(wbar_in, ghost, plane, ny, nx, bc);
     });
 }
 

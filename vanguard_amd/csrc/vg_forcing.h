@@ -78,8 +78,8 @@ __device__ __forceinline__ void fractional_step(const typename P::Params &m, con
     // checked by itself: of the last steps only the fields are computed that the few
     // source slots need, and a check over all fields would keep the others alive.  The
     // 17-field kernel, whose code is twice the instruction cache, keeps one division
-    // (HPR 640 x 512: 285 us a launch, 309 with the short one beside it, 302 with the
-    // pieces by selects).
+    // (HPR 640 x 512: 269 us a launch; when it was 285, 309 with the short one beside
+    // it and 302 with the pieces by selects).
     const double cl = 0.5 * (1.0 + bias), cr = 0.5 * (1.0 - bias);
     const double f1 = limiter_value(1.0, bias, limiter);
     const bool bias_in_range = (bias >= -1.0) && (bias <= 1.0);
@@ -190,7 +190,7 @@ __device__ __forceinline__ void forcing_cell(const typename P::Params &m, const 
     // Nine fields: the stages stay a loop, a third of the code (unrolled, 88 KB against
     // the instruction cache's 64: 38.3 us a launch on 384 x 384, 37.3 in the loop).
     // Seventeen: a loop holds all increments over every predictor (229
-    // registers spilled instead of 57, 347 us a launch on 640 x 512 instead of 285).
+    // registers spilled instead of 57, 347 us a launch on 640 x 512 against 285).
     if constexpr (NF <= 9) {
 #pragma clang loop unroll(disable)
         for (int st = 0; st < 4; st++) stage(st);

@@ -113,14 +113,15 @@ __global__ __launch_bounds__(256) void constant_planes_kernel(const double *__re
 // reads of halos and partial lines count: HPR 1024 x 1024 (285 MB) 209.6 / 235.8 and
 // 187.7 / 211.8, Euler 4096 x 4096 407 / 537 and 408 / 438.  The line is drawn at
 // the bytes one sweep reads and writes, between the two; the sweeps with little
-// arithmetic to hide the reads behind (FORCE, FAST mode) meet it earlier: FAST
-// 850 x 850 (69 MB) 29.0 / 22.5, 1531 x 1000 (147 MB) 27.8 / 31.9.
+// arithmetic to hide the reads behind (FAST mode, FORCE) meet it earlier: FAST x 850 x
+// 850 (69 MB) 29.0 / 22.5, 1531 x 1000 (147 MB) 27.8 / 31.9; FORCE y 700 x 700 (47 MB)
+// 22.4 / 15.9, 850 x 850 24.0 / 26.3.
 template <class P>
 bool small_tiles(int order, int mode, int ny, int nx)
 {
     const long long bytes = 2LL * StoredFields<P>::n * 8 * ny * nx;
-    const long long most = (order == 2 && mode == VG_MODE_EXACT) ? 160LL << 20 : 96LL << 20;
-    return bytes <= most && ny <= 65535;   // ny: one row per block in the launch's second dimension
+    const long long mb = (order == 1) ? 48 : (mode == VG_MODE_EXACT ? 160 : 96);
+    return bytes <= mb << 20 && ny <= 65535;   // ny: one row per block in the launch's second dimension
 }
 
 // Blocks of an x sweep, and its launch.
@@ -713,6 +714,7 @@ struct GridState {
         VG_HIP(hipEventCreate(&e1));
         VG_HIP(hipEventRecord(e0, ctx->stream));
         const int start_cur = cur;
+        int graph_steps = 0;   // steps enqueued as replays, before any one by one
         // Steps to enqueue before the clock is read again: what is left of the step
         // cap, and of the way to the final time at the last step's length (before
         // the start-up ramp is over, at the one its wave speed gives), so that few
@@ -739,7 +741,8 @@ struct GridState {
                    std::to_string(limiter) + "|" + std::to_string((unsigned long long)(uintptr_t)dlog) + "|" +
                    std::to_string(dt_cap) + "|" + std::to_string(subcycles) + "|" + std::to_string(y_variant) + "|" +
                    std::to_string(cur) + "|" + std::to_string(n_partials) + "|" + std::to_string((int)reduced);
-            if (!graph || key != graph_key) {
+            auto capture = [&]() -> int {
+                if (graph && key == graph_key) return VG_OK;
                 if (graph) {
                     hipGraphExecDestroy(graph);
                     graph = nullptr;
@@ -767,10 +770,29 @@ struct GridState {
                     return VG_ERR_HIP;
                 }
                 graph_key = key;
-            }
+                return VG_OK;
+            };
             for (;;) {
-                const int reps = (steps_left() + kGraphSteps - 1) / kGraphSteps;
+                const int left = steps_left();
+                int reps = left / kGraphSteps, rest = left % kGraphSteps;
+                // The last few steps before the step cap run one by one: a replay would
+                // find the clock stopped for the rest of its steps (a launch of which
+                // costs 2 us doing nothing), and a run of only those needs no graph.
+                const bool last = max_steps > 0 && left == max_steps - h.steps_this_run;
+                if (rest > 0 && !(last && rest <= kGraphSteps / 2)) {
+                    reps += 1;
+                    rest = 0;
+                }
+                if (reps > 0) {
+                    int rc = capture();
+                    if (rc) return rc;
+                }
                 for (int r = 0; r < reps; r++) VG_HIP(hipGraphLaunch(graph, ctx->stream));
+                graph_steps += reps * kGraphSteps;
+                for (int s = 0; s < rest; s++) {
+                    int rc = enqueue_step<ORDER, MODE>(bc, dx, bias, limiter, m, dlog, dt_cap);
+                    if (rc) return rc;
+                }
                 VG_HIP(hipMemcpyAsync(&h, clk, sizeof(Clock), hipMemcpyDeviceToHost, ctx->stream));
                 VG_HIP(hipStreamSynchronize(ctx->stream));
                 if (h.done) break;
@@ -789,7 +811,8 @@ struct GridState {
                 if (max_steps > 0 && h.steps_this_run >= max_steps) break;
             }
         }
-        const bool two_sets = ctx->graphs && !ctx->timing && begins_in_sweep(ORDER, MODE, m);
+        // a run that ended inside its replays may have left its keys in the second set
+        const bool two_sets = graph_steps >= h.steps_this_run && graph_steps > 0 && begins_in_sweep(ORDER, MODE, m);
         clock_finish_kernel<<<1, 256, 0, ctx->stream>>>(clk, two_sets ? partials : nullptr, slots, n_partials);
         int rc = launch_status("clock_finish");
         if (rc) return rc;

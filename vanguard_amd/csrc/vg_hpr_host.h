@@ -46,9 +46,6 @@ inline HPRParams hpr_to_params(const vg_hpr_params *p)
     m.cs2 = m.cs * m.cs;
     m.a2 = m.alpha * m.alpha;
     m.c02 = m.c0 * m.c0;
-    m.inv_G = 1.0 / m.G;
-    m.inv_Gcv = 1.0 / (m.G * m.cv);
-    m.short_div = scale_in_range(m.G) && scale_in_range(m.G * m.cv);
     return m;
 }
 

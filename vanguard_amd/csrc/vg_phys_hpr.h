@@ -29,10 +29,6 @@ struct HPRParams {
     double G, cs2, a2;
     int eos;
     double p_ref, c0, gamma0, s_h, alpha_gr, sigma_y, n_pow, c02;
-    // reciprocals of G and G cv, estimates only (quot_near), and whether both are
-    // scales it takes
-    double inv_G, inv_Gcv;
-    int short_div;
 };
 
 // EOS: the equation of state, fixed per kernel (0 StiffenedGas, 1
@@ -146,30 +142,6 @@ struct HPRPhysT {
     }
     __device__ static __forceinline__ double mg_T_p(const Params &m, double rho) { return mg_e_p(m, rho) / m.cv; }
 
-    // The same, given the shared divisor d of rho: the stiffened gas divides by rho,
-    // rho Gamma and rho Gamma cv, whose reciprocals come from rho's where in range.
-    __device__ static __forceinline__ bool short_div(const Params &m, const SharedDivisor &d)
-    {
-        return EOS == 0 && d.fast && m.short_div;
-    }
-    __device__ static __forceinline__ double mg_e_d(const Params &m, double rho, double p, const SharedDivisor &d)
-    {
-        if (short_div(m, d))
-            return quot_refined(m.p_inf, d) + quot_near(p - mg_pref(m, rho), rho * m.G, d.y * m.inv_G);
-        return mg_e(m, rho, p);
-    }
-    __device__ static __forceinline__ double mg_p_d(const Params &m, double rho, double e, const SharedDivisor &d)
-    {
-        if (EOS == 0) return ((e - quot(m.p_inf, d)) * rho * m.G) + mg_pref(m, rho);
-        return mg_p(m, rho, e);
-    }
-    __device__ static __forceinline__ double mg_T_d(const Params &m, double rho, double p, const SharedDivisor &d)
-    {
-        if (short_div(m, d))
-            return m.t_ref + quot_near(p - mg_pref(m, rho), rho * m.G * m.cv, d.y * m.inv_Gcv);
-        return mg_T(m, rho, p);
-    }
-
     // ---- 3x3 helpers (Mathematics/matrixalgebra.cpp, tensoralgebra.cpp) ------------
     template <int NN>
     __device__ static __forceinline__ void load_A(const double (&s)[NN], double (&A)[3][3])
@@ -260,12 +232,11 @@ struct HPRPhysT {
         return 0.5 * ((u * u) + (v * v) + (w * w));
     }
     __device__ static __forceinline__ double pressure_of(const Params &m, double rho, double E, double u, double v, double w,
-                                                         const double (&A)[3][3], double jx, double jy, double jz,
-                                                         const SharedDivisor &d)
+                                                         const double (&A)[3][3], double jx, double jy, double jz)
     {
         double e = E - (e_macro(u, v, w) + e_dist(m, A));
         if (m.is_thermal) e -= e_therm(m, jx, jy, jz);
-        return mg_p_d(m, rho, e, d);
+        return mg_p(m, rho, e);
     }
     // c_s^2 (A dev(A^T A)) (hprderivatives.cpp:17-24) and the shear stress
     // -rho A^T E_A with its density derivative -1 * A^T E_A (hprequationofstate.cpp:55-81).
@@ -292,16 +263,10 @@ struct HPRPhysT {
     // computeConservedVariableVector (hprstatevector.cpp:105-132).
     __device__ static __forceinline__ void prim_to_cons(const Params &m, const double (&w)[NF], double (&U)[NF])
     {
-        prim_to_cons_d(m, w, shared_divisor(w[0]), U);
-    }
-    // ... given the shared divisor of rho.
-    __device__ static __forceinline__ void prim_to_cons_d(const Params &m, const double (&w)[NF],
-                                                          const SharedDivisor &d, double (&U)[NF])
-    {
         double A[3][3];
         load_A(w, A);
         const double rho = w[0];
-        double E = mg_e_d(m, rho, w[1], d) + e_dist(m, A) + e_macro(w[11], w[12], w[13]);
+        double E = mg_e(m, rho, w[1]) + e_dist(m, A) + e_macro(w[11], w[12], w[13]);
         if (m.is_thermal) E += e_therm(m, w[14], w[15], w[16]);
         U[0] = rho;
         U[1] = rho * E;
@@ -356,7 +321,7 @@ struct HPRPhysT {
         }
         const double E = q[6];
         w[0] = rho;
-        w[1] = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz, d);
+        w[1] = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz);
 #pragma unroll
         for (int k = 2; k < 11; k++) w[k] = U[k];
         w[11] = u;
@@ -389,7 +354,7 @@ struct HPRPhysT {
         const double jy = m.is_thermal ? q[4] : 0.0;
         const double jz = m.is_thermal ? q[5] : 0.0;
         const double E = q[6];
-        const double p = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz, d);
+        const double p = pressure_of(m, rho, E, u, v, z, A, jx, jy, jz);
 #pragma unroll
         for (int k = 0; k < NF; k++) F[k] = 0.0;
         const double vn = (DIR == 0) ? u : v;
@@ -415,7 +380,7 @@ struct HPRPhysT {
             F[2 + 3 * i + DIR] = s;
         }
         if (m.is_thermal) {
-            const double T = mg_T_d(m, rho, p, d);
+            const double T = mg_T(m, rho, p);
             F[1] = F[1] + (T * (m.a2 * (DIR == 0 ? jx : jy)));
             F[14] = rho * (vn * jx);
             F[15] = rho * (vn * jy);
@@ -425,7 +390,10 @@ struct HPRPhysT {
     }
 
     // setConservedVariableVector of x, then the conserved vector and flux of that
-    // state: rho comes back unchanged, so all three share its divisor.
+    // state: rho comes back unchanged, so the quotients by it share its divisor.  The
+    // energies' few other divisions stay the compiler's: with short ones taken by a
+    // range check the relaxation kernel, bound by its code's size as much as by its
+    // arithmetic, ran 0.81 ms on 1024 x 1024 instead of 0.76.
     template <int DIR>
     __device__ static __forceinline__ void round_trip(const Params &m, const double (&x)[NF], double (&U)[NF],
                                                       double (&F)[NF])
@@ -433,7 +401,7 @@ struct HPRPhysT {
         const SharedDivisor d = shared_divisor(x[0]);
         double w[NF];
         cons_to_prim_d(m, x, d, w);
-        prim_to_cons_d(m, w, d, U);
+        prim_to_cons(m, w, U);
         flux_of<DIR>(m, U, d, F);
     }
 
@@ -597,8 +565,8 @@ struct HPRPhysT {
             double q[7];
             by_rho(U, d, q);
             const double jx = q[3], jy = q[4], jz = q[5];
-            const double p = pressure_of(m, rho, q[6], q[0], q[1], q[2], A, jx, jy, jz, d);
-            const double T = mg_T_d(m, rho, p, d);
+            const double p = pressure_of(m, rho, q[6], q[0], q[1], q[2], A, jx, jy, jz);
+            const double T = mg_T(m, rho, p);
             const double th2 = 1.0 / (m.a2 * m.tau2 * ((rho / m.rho0) * (m.t0 / T)));
             S[14] = -rho * th2 * (m.a2 * jx);
             S[15] = -rho * th2 * (m.a2 * jy);

@@ -127,29 +127,24 @@ VG_QUOT_FN double quot(double a, const SharedDivisor &d)
 }
 
 #ifdef __HIPCC__
-// RN(a / b) from an estimate y of 1 / b a few units off in the last place (b and a in
-// quot_refined's range): one Newton step gives the estimate that two give from the
-// hardware's, and the quotient ends as it does there.
-__device__ __forceinline__ double quot_near(double a, double b, double y)
+// RN(a / (c * d.b)) for a scale c with 2^-20 <= c <= 2^20 whose reciprocal is
+// c_inv, d.fast, and a in quot_refined's range: d's reciprocal times c_inv is within
+// two units of 1 / (c * d.b) in the last place, so one Newton step gives the
+// estimate that two give from the hardware's, and the quotient ends as it does
+// there.  Six instructions where the division sequence takes its own reciprocal.
+__device__ __forceinline__ double quot_scaled(double a, const SharedDivisor &d, double c, double c_inv)
 {
+    const double b = c * d.b;
+    double y = d.y * c_inv;
     const double e = __builtin_fma(-b, y, 1.0);
     y = __builtin_fma(y, e, y);
     return div_finish(a, b, y);
 }
 
-// RN(a / (c * d.b)) for a scale c with 2^-20 <= c <= 2^20 whose reciprocal is
-// c_inv, and d.fast: d's reciprocal times c_inv is within two units of
-// 1 / (c * d.b) in the last place.  Six instructions where the division sequence
-// takes its own reciprocal.
-__device__ __forceinline__ double quot_scaled(double a, const SharedDivisor &d, double c, double c_inv)
-{
-    return quot_near(a, c * d.b, d.y * c_inv);
-}
-
 // RN(a / 3) for a zero or 2^-1000 <= |a| <= 2^1000 (a NaN for an infinite a).
 __device__ __forceinline__ double third(double a) { return div_finish(a, 3.0, 1.0 / 3.0); }
 // Whether c is a scale quot_scaled takes.
-__host__ __device__ inline bool scale_in_range(double c) { return (c >= 0x1p-20) && (c <= 0x1p+20); }
+__device__ __forceinline__ bool scale_in_range(double c) { return (c >= 0x1p-20) && (c <= 0x1p+20); }
 #endif
 
 // q[k] = RN(a[k] / d.b) for a group of numerators sharing the divisor: one

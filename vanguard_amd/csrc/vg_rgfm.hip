@@ -487,8 +487,10 @@ struct RGFMGrid {
                 }
                 graph_key = key;
             }
-            const int reps = std::max(1, chunk / kGraphSteps);
             for (;;) {
+                // no more replays than the step cap leaves
+                const int left = max_steps > 0 ? std::min(chunk, max_steps - h.steps_this_run) : chunk;
+                const int reps = std::max(1, (left + kGraphSteps - 1) / kGraphSteps);
                 for (int r = 0; r < reps; r++) VG_HIP(hipGraphLaunch(graph, s));
                 VG_HIP(hipMemcpyAsync(&h, clk, sizeof(Clock), hipMemcpyDeviceToHost, s));
                 VG_HIP(hipStreamSynchronize(s));
