@@ -90,7 +90,7 @@ int vg_ctx_reset_timing(vg_ctx *ctx);
  * reference counterpart (the reference has no device). */
 int vg_ctx_set_graphs(vg_ctx *ctx, int enabled);
 /* Tile-shape autotuner (default on): the first run on a grid shape times the
- * candidate y-sweep shapes (threads per block x rows per strip) on that grid
+ * candidate y-sweep shapes (walked strips of rows, or tiles) on that grid
  * and keeps the fastest for the context.  vg_ctx_tuned_shape returns the chosen
  * variant for a key "physics/order/mode/ny/nx" (forward Y sweeps, variants 0-7;
  * physics "euler", or "euler_planar" for grids swept with 4 fields)
