@@ -98,7 +98,10 @@ int vg_ctx_set_graphs(vg_ctx *ctx, int enabled);
  * 0-5; "euler_planar_adjoint_..." for the 4-field adjoint sweeps; a 1D grid of n
  * cells has ny = 1, nx = n), -1 if not tuned
  * yet.  vg_ctx_set_tuned_shape pins a variant for a key (for example one saved
- * from an earlier process); -1 forgets it.  Shapes change speed, never results. */
+ * from an earlier process); -1 forgets it.  The forward X sweeps' shape follows from
+ * the grid's size and is not tuned; "physics/order/mode/ny/nx/x" pins it (0: walked
+ * rows, 1: tiles; "rgfm_physics/..." for the two-material RGFM grids).  Shapes change
+ * speed, never results. */
 int vg_ctx_set_autotune(vg_ctx *ctx, int enabled);
 /* Constant-field specialisation (default on): an Euler grid whose out-of-plane
  * velocity is +0 and reaction progress exactly 1 in every cell (checked at the

@@ -102,26 +102,37 @@ __global__ __launch_bounds__(256) void constant_planes_kernel(const double *__re
 
 // ---- sweep shapes ----------------------------------------------------------------
 
-// Whether a grid's sweeps take small tiles of one cell per thread.  A block that
-// walks rows (sweep_x_kernel with several rows, sweep_y_kernel) computes no halo
-// twice and reads whole cache lines, but runs its rows one after another: with too
-// few blocks to fill the device the sweep takes as long as one walk.  Measured per
-// sweep, x walk / x tile and y walk / y tile (EXACT SLIC): Euler 200 x 200 13.9 /
-// 5.1 us and 41.9 / 5.4 us, 1024 x 1024 39.1 / 32.3 and 49.9 / 34.9; MHD 384 x 384
-// 25.4 / 15.7 and 79.0 / 16.5, 1024 x 1024 (151 MB) 80.0 / 72.1 and 85.5 / 75.0; HPR
-// 640 x 512 (89 MB) 105.7 / 79.5 and 186.6 / 75.8.  Beyond the cache the tiles' extra
-// reads of halos and partial lines count: HPR 1024 x 1024 (285 MB) 209.6 / 235.8 and
-// 187.7 / 211.8, Euler 4096 x 4096 407 / 537 and 408 / 438.  The line is drawn at
-// the bytes one sweep reads and writes, between the two; the sweeps with little
-// arithmetic to hide the reads behind (FAST mode, FORCE) meet it earlier: FAST x 850 x
-// 850 (69 MB) 29.0 / 22.5, 1531 x 1000 (147 MB) 27.8 / 31.9; FORCE y 700 x 700 (47 MB)
-// 22.4 / 15.9, 850 x 850 24.0 / 26.3.
+// Whether a grid's sweeps along dir take small tiles of one cell per thread.  A block
+// that walks rows (sweep_x_kernel with several rows, sweep_y_kernel) computes no halo
+// twice and reads whole cache lines, but runs its rows one after another: with too few
+// blocks to fill the device the sweep takes as long as one walk.  Beyond the cache the
+// tiles' extra reads of halos and partial lines count instead.  So the line is drawn at
+// the bytes a sweep reads and writes: the planes that P, the physics in use, carries
+// (four where a reduced one sweeps).
+//   y, microseconds a sweep, walk / tile.  EXACT SLIC: 4 fields 12 MB 42.5 / 14.1, 90 MB
+//     56.4 / 41.5, 150 MB 69.6 / 57.6, 170 MB 71.7 / 73.2; 6 fields 150 MB 78.6 / 62.2; 9
+//     fields 130 MB 73 / 64; 17 fields 60 MB 159 / 57, 150 MB 163 / 92.  The sweeps with
+//     little arithmetic to hide the reads behind meet it earlier.  FAST SLIC: 4 fields 40 MB
+//     31.7 / 20.7, 90 MB 40.0 / 36.6, 140 MB 52.9 / 61.0.  FORCE EXACT: 4 fields 46 MB 23.8 /
+//     18.1, 55 MB 23.8 / 25.1; FAST: 30 MB 15.9 / 14.9, 38 MB 16.1 / 18.5.
+//   x, microseconds a step of three sweeps, x walks / x tiles.  EXACT SLIC: 9 fields 150 MB
+//     269 / 232, 200 MB 310 / 307; 17 fields 150 MB 390 / 280; 6 fields 60 MB 107 / 93, 90 to
+//     150 MB within 10 % either way by the shape, 170 MB 210 / 219; 4 fields, where the
+//     walk's limiter skips most of the divisions, 40 MB 77.0 / 70.1, 60 to 75 MB by the shape
+//     86 / 93 (1982 x 495) to 106 / 94 (2090 x 522), 90 MB 118 / 129, 110 MB 141 / 151.  FAST SLIC: 4 fields 60 MB 75.1 / 73.2, 90 MB 109 / 101 to 98 / 97, 130 MB 130 /
+//     130; 6 fields 60 MB 88 / 76.  FORCE: 4 fields EXACT 30 MB 42.9 / 40.7, 36 MB 41.9 / 41.6,
+//     48 MB 54.3 / 55.2, FAST 48 MB 42.8 / 44.7; 6 fields EXACT 48 MB 52.4 / 50.5, FAST 30 MB
+//     37.6 / 37.2, 42 MB 41.7 / 44.9; 9 fields 46 MB 62.7 / 58.3.
 template <class P>
-bool small_tiles(int order, int mode, int ny, int nx)
+bool small_tiles(int dir, int order, int mode, int ny, int nx)
 {
+    if (ny > 65535) return false;   // one row per block in the launch's second dimension
     const long long bytes = 2LL * StoredFields<P>::n * 8 * ny * nx;
-    const long long mb = (order == 1) ? 48 : (mode == VG_MODE_EXACT ? 160 : 96);
-    return bytes <= mb << 20 && ny <= 65535;   // ny: one row per block in the launch's second dimension
+    const bool exact = mode == VG_MODE_EXACT;
+    long long mb;
+    if (dir == 0) mb = (order == 2) ? (!exact ? 96 : P::NF <= 4 ? 80 : 160) : (P::NF <= (exact ? 4 : 6) ? 36 : 48);
+    else mb = (order == 2) ? (exact ? 160 : 96) : (exact ? 48 : 32);
+    return bytes <= mb << 20;
 }
 
 // Blocks of an x sweep, and its launch.
@@ -167,7 +178,7 @@ void launch_y_tile(hipStream_t s, const SweepArgs<P> &a)
 template <class P>
 int default_y(int order, int mode, int ny, int nx)
 {
-    return small_tiles<P>(order, mode, ny, nx) ? 4 : 0;
+    return small_tiles<P>(1, order, mode, ny, nx) ? 4 : 0;
 }
 
 template <class P, int ORDER, int MODE>
@@ -202,9 +213,10 @@ inline std::string tune_key(const char *phys, int order, int mode, int ny, int n
 }
 
 // Picks the y-sweep shape for a grid: the context's table when the shape was
-// tuned before; default_y's where nothing is tuned; otherwise each candidate runs once to warm up and some times
-// timed on the caller's grid (a.in -> a.out, with a.clk a scratch clock holding
-// a small positive dt, no CFL fusion), and the fastest is recorded.
+// tuned before; default_y's where nothing is tuned; otherwise each candidate runs once
+// to warm up and some times timed on the caller's grid (a.in -> a.out, with a.clk a
+// scratch clock holding a small positive dt, no CFL fusion), and the fastest is
+// recorded.
 template <class P, int ORDER, int MODE>
 int tune_y(vg_ctx *ctx, const std::string &key, SweepArgs<P> a, int &variant)
 {
@@ -219,10 +231,11 @@ int tune_y(vg_ctx *ctx, const std::string &key, SweepArgs<P> a, int &variant)
     hipEvent_t e0, e1;
     VG_HIP(hipEventCreate(&e0));
     VG_HIP(hipEventCreate(&e1));
-    // Where the small tiles are the rule only they are candidates: on such a grid the
-    // walks are two to twenty times slower, and the tiles' few microseconds want more
-    // runs to tell apart (MHD 384 x 384, 14.2 us against 20, was mistaken with three).
-    const bool small = small_tiles<P>(ORDER, MODE, a.ny, a.nx);
+    // Where the small tiles are the rule only they are candidates: the walks are as fast to
+    // 1.3 times slower at its line (above) and two to eight times slower on small grids,
+    // and more runs tell the two tiles' few microseconds apart (MHD 384 x 384, 14.2 us
+    // against 20, was mistaken with three).
+    const bool small = small_tiles<P>(1, ORDER, MODE, a.ny, a.nx);
     const int v0 = small ? 4 : 0, v1 = small ? 6 : kYVariants, runs = small ? 10 : 3;
     float best = 0.0f;
     for (int v = v0; v < v1; v++) {
@@ -245,11 +258,21 @@ int tune_y(vg_ctx *ctx, const std::string &key, SweepArgs<P> a, int &variant)
     return VG_OK;
 }
 
+// Whether a grid's x sweeps are tiles: as pinned in the context's table (key: the y
+// sweep's and "/x"; 0 walks, 1 tiles), else small_tiles' choice.
+template <class P>
+bool tiles_in_x(const vg_ctx *ctx, int order, int mode, int ny, int nx)
+{
+    auto it = ctx->tuned.find(tune_key(P::name, order, mode, ny, nx) + "/x");
+    if (it == ctx->tuned.end()) return small_tiles<P>(0, order, mode, ny, nx);
+    return it->second == 1 && ny <= 65535;
+}
+
 template <class P>
 struct GridState {
     static constexpr int NF = P::NF;
     static constexpr int NS = StoredFields<P>::n;   // planes per buffer (stored fields per cell)
-        vg_ctx *ctx = nullptr;
+    vg_ctx *ctx = nullptr;
     int dim = 2, ny = 1, nx = 1;
     long long plane = 0, cells = 0;
     double *buf[2] = {nullptr, nullptr};
@@ -410,12 +433,22 @@ struct GridState {
         return VG_OK;
     }
 
+    // Whether the x sweeps, with the physics of this run, are tiles.
+    bool x_tiles(int order, int mode) const
+    {
+        using R = typename ReducedPhys<P>::type;
+        if constexpr (!std::is_void_v<R>) {
+            if (reduced) return tiles_in_x<R>(ctx, order, mode, ny, nx);
+        }
+        return tiles_in_x<P>(ctx, order, mode, ny, nx);
+    }
+
     // Blocks of the launch that ends a step and folds in the next step's CFL
     // maximum: the last source sub-cycle, else the last x sweep.
     int fused_count(int order, int mode = VG_MODE_EXACT) const
     {
         if (SourceStage<P>::kActive && subcycles > 0 && order == 2) return (int)SourceStage<P>::blocks(*this);
-        const bool tiles = small_tiles<P>(order, mode, ny, nx);
+        const bool tiles = x_tiles(order, mode);
         const dim3 g = (order == 2) ? x_blocks<P, 2>(tiles, ny, nx) : x_blocks<P, 1>(tiles, ny, nx);
         return (int)(g.x * g.y);
     }
@@ -476,12 +509,12 @@ struct GridState {
                 if (begin)
                     sweep_x_begin_kernel<Q, ORDER, MODE><<<x_blocks<Q, ORDER>(true, ny, nx), kWave, 0, ctx->stream>>>(
                         a, *begin);
-                else launch_x<Q, ORDER, MODE>(ctx->stream, small_tiles<P>(ORDER, MODE, ny, nx), a);
+                else launch_x<Q, ORDER, MODE>(ctx->stream, x_tiles(ORDER, MODE), a);
             });
         }
         // The y sweep never ends a step, so it never writes the CFL partials.
         a.fuse_max = 0;
-        return launch_y<Q, ORDER, MODE>(ctx, y_variant >= 0 ? y_variant : default_y<P>(ORDER, MODE, ny, nx), a);
+        return launch_y<Q, ORDER, MODE>(ctx, y_variant >= 0 ? y_variant : default_y<Q>(ORDER, MODE, ny, nx), a);
     }
 
     template <int ORDER, int MODE>
@@ -571,7 +604,7 @@ struct GridState {
     bool begins_in_sweep(int order, int mode, const typename P::Params &m) const
     {
         if (order == 2 && ((SourceStage<P>::kActive && subcycles > 0) || PostStep<P>::active(m))) return false;
-        return n_partials <= kBeginSlots && small_tiles<P>(order, mode, ny, nx);
+        return n_partials <= kBeginSlots && x_tiles(order, mode);
     }
 
     // One step.  `captured`: the step is recorded into a graph whose steps come in
@@ -740,7 +773,8 @@ struct GridState {
             key += "|" + std::to_string(ORDER) + "|" + std::to_string(MODE) + "|" + std::to_string(bc) + "|" +
                    std::to_string(limiter) + "|" + std::to_string((unsigned long long)(uintptr_t)dlog) + "|" +
                    std::to_string(dt_cap) + "|" + std::to_string(subcycles) + "|" + std::to_string(y_variant) + "|" +
-                   std::to_string(cur) + "|" + std::to_string(n_partials) + "|" + std::to_string((int)reduced);
+                   std::to_string(cur) + "|" + std::to_string(n_partials) + "|" + std::to_string((int)reduced) + "|" +
+                   std::to_string((int)x_tiles(ORDER, MODE));
             auto capture = [&]() -> int {
                 if (graph && key == graph_key) return VG_OK;
                 if (graph) {

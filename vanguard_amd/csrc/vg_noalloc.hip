@@ -107,7 +107,7 @@ int launch_noalloc(hipStream_t s, double *base, double *cells, const double *wit
     args.clk = clk;
     args.partials = nullptr;
     args.fixed_params = 1;
-    const bool tiles = vg::small_tiles<P>(ORDER, MODE, gy, gx);
+    const bool tiles = vg::small_tiles<P>(dir, ORDER, MODE, gy, gx);
     if (dir == 0) vg::launch_x<P, ORDER, MODE>(s, tiles, args);
     else if (tiles) vg::launch_y_tile<P, ORDER, MODE, 256, 8>(s, args);
     else vg::launch_y_walk<P, ORDER, MODE, vg::Tiles<P>::bsy, vg::Tiles<P>::hy>(s, args);

@@ -42,7 +42,7 @@ struct RGFMGrid {
     Clock *clk = nullptr, *tune_clk = nullptr;
     unsigned long long *partials = nullptr;
     int max_blocks = 0, circ_blocks = 0;
-    int y_variant = 0;                  // y-sweep shape (default_y, or autotuned)
+    int y_variant = -1;                 // y-sweep shape, autotuned (-1: default_y)
     bool reduced = false;               // this run sweeps with the 4-field EulerPlanarPhys
     int *flag = nullptr;                // constant-plane check result
     hipGraphExec_t graph = nullptr;     // captured chunk of steps
@@ -57,7 +57,6 @@ struct RGFMGrid {
         nx = x;
         cells = (long long)ny * nx;
         plane = (cells + 63) / 64 * 64;
-        y_variant = default_y<EulerPhys>(2, VG_MODE_EXACT, ny, nx);
         for (int b = 0; b < 2; b++) {
             VG_HIP(hipMalloc(&m1[b], sizeof(double) * 6 * plane));
             VG_HIP(hipMalloc(&m2[b], sizeof(double) * 6 * plane));
@@ -185,19 +184,42 @@ struct RGFMGrid {
         const SweepArgs<Q> a = sweep_args<Q>(in, out, scale, h, bias, limiter, m);
         if (dir == 0) {
             return ctx->timed("rgfm_sweep_x",
-                              [&] { launch_x<Q, 2, MODE>(ctx->stream, small_tiles<EulerPhys>(2, MODE, ny, nx), a); });
+                              [&] { launch_x<Q, 2, MODE>(ctx->stream, x_tiles(MODE), a); });
         }
-        return launch_y<Q, 2, MODE>(ctx, y_variant, a);
+        return launch_y<Q, 2, MODE>(ctx, y_shape<Q>(MODE), a);
     }
 
-    // Both materials' sweeps in one direction, in one launch where the grid's sweeps
-    // are small tiles (320 x 640: x 19.6 us in two launches, 14.0 in one; y 22.2, 15.8).
+    template <class Q>
+    int y_shape(int mode) const
+    {
+        return y_variant >= 0 ? y_variant : default_y<Q>(2, mode, ny, nx);
+    }
+
+    // Whether the x sweeps, with the physics of this run, are tiles: the context's table
+    // (key: as an Euler grid's, "rgfm_" before it), else up to 160 MB read and written per
+    // material.  Both materials in one launch keep the tiles ahead of the walks, two
+    // launches, for longer than a single Euler grid's (microseconds a step, walks / tiles:
+    // 320 x 640 123 / 96, 1024 x 1024 251 / 226, 1024 x 2048 423 / 414; 6 fields 1024 x 1600,
+    // 150 MB, 464 / 447).
+    template <class Q>
+    bool x_tiles_as(int mode) const
+    {
+        auto it = ctx->tuned.find("rgfm_" + tune_key(Q::name, 2, mode, ny, nx) + "/x");
+        if (ny > 65535) return false;
+        if (it != ctx->tuned.end()) return it->second == 1;
+        return 2LL * Q::NF * 8 * cells <= 160LL << 20;
+    }
+    bool x_tiles(int mode) const { return reduced ? x_tiles_as<EulerPlanarPhys>(mode) : x_tiles_as<EulerPhys>(mode); }
+
+    // Both materials' sweeps in one direction, in one launch where that direction's
+    // sweeps are tiles (320 x 640: x 19.6 us in two launches, 14.0 in one; y 22.2, 15.8).
     template <class Q, int MODE>
     int sweep_both_as(int dir, const double *in1, double *out1, const double *in2, double *out2, double scale, double h,
                       double bias, int limiter, const EP &p1, const EP &p2)
     {
-        const bool tiles = small_tiles<EulerPhys>(2, MODE, ny, nx);
-        if (dim == 2 && tiles && (dir == 0 || y_variant == 4 || y_variant == 5)) {
+        const int yv = y_shape<Q>(MODE);
+        const bool y_tiles = (yv == 4 || yv == 5) && ny <= 28 * 65535;   // as launch_y
+        if (dim == 2 && (dir == 0 ? x_tiles(MODE) : y_tiles)) {
             const SweepPair<Q> p = {sweep_args<Q>(in1, out1, scale, h, bias, limiter, p1),
                                     sweep_args<Q>(in2, out2, scale, h, bias, limiter, p2)};
             const hipStream_t s = ctx->stream;
@@ -206,7 +228,7 @@ struct RGFMGrid {
                     dim3 grid = x_blocks<Q, 2>(true, ny, nx);
                     grid.z = 2;
                     sweep_x_pair_kernel<Q, 2, MODE><<<grid, kWave, 0, s>>>(p);
-                } else if (y_variant == 4) {
+                } else if (yv == 4) {
                     sweep_y_tile_pair_kernel<Q, 2, MODE, 256, 8><<<dim3((nx + 7) / 8, (ny + 27) / 28, 2), 256, 0, s>>>(p);
                 } else {
                     sweep_y_tile_pair_kernel<Q, 2, MODE, 512, 8><<<dim3((nx + 7) / 8, (ny + 59) / 60, 2), 512, 0, s>>>(p);
@@ -459,7 +481,7 @@ struct RGFMGrid {
             key += "|" + std::to_string(riemann) + "|" + std::to_string(mode) + "|" + std::to_string(limiter) + "|" +
                    std::to_string((unsigned long long)(uintptr_t)dlog) + "|" + std::to_string(dt_cap) + "|" +
                    std::to_string(y_variant) + "|" + std::to_string(cur) + "|" + std::to_string(pcur) + "|" +
-                   std::to_string((int)reduced);
+                   std::to_string((int)reduced) + "|" + std::to_string((int)x_tiles(mode));
             if (!graph || key != graph_key) {
                 if (graph) {
                     hipGraphExecDestroy(graph);

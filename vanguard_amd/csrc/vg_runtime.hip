@@ -235,9 +235,12 @@ int vg_ctx_release_workspace(vg_ctx *ctx)
 int vg_ctx_set_tuned_shape(vg_ctx *ctx, const char *key, int variant)
 {
     VG_CHECK(ctx != nullptr && key != nullptr, "vg_ctx_set_tuned_shape: null argument");
-    const bool adjoint = std::string(key).find("adjoint") != std::string::npos;
-    VG_CHECK(variant >= -1 && variant < (adjoint ? 6 : 8),
+    const std::string k(key);
+    const bool adjoint = k.find("adjoint") != std::string::npos;
+    const bool x = k.size() >= 2 && k.compare(k.size() - 2, 2, "/x") == 0;
+    VG_CHECK(variant >= -1 && variant < (adjoint ? 6 : x ? 2 : 8),
              adjoint ? "vg_ctx_set_tuned_shape: adjoint variant must be -1..5"
+             : x     ? "vg_ctx_set_tuned_shape: x-sweep variant must be -1..1"
                      : "vg_ctx_set_tuned_shape: y-sweep variant must be -1..7");
     if (variant < 0) ctx->tuned.erase(key);
     else ctx->tuned[key] = variant;
