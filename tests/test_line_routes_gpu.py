@@ -31,26 +31,29 @@ def _mhd(n, seed=0):
 
 
 # 252 / 253: one tile of 256 threads or of 512; 508 / 509 (SLIC) and 1020 / 1021
-# (FORCE): the last workgroup size and the first grid size; 60 / 124: MHD tiles.
-@pytest.mark.parametrize("n", [60, 124, 125, 252, 253, 508, 509, 569, 1020, 1021])
+# (FORCE): the last size of a long run in one workgroup and the first on the grid path;
+# 60 / 124: MHD tiles.  Up to 12 steps (SLIC) the workgroup keeps an Euler line of two
+# tiles; 11 steps of 2100 cells are launched one by one, 41 steps replayed.
+@pytest.mark.parametrize("n", [60, 124, 125, 252, 253, 508, 509, 569, 1020, 1021, 2100])
 @pytest.mark.parametrize("order", [2, 1])
-def test_1d_routes_match_oracle(vg_ctx, n, order):
-    kw = dict(order=order, dim=1, dx=1.0 / n, cfl=0.7, tfinal=math.inf, max_steps=11, bias=0.0, limiter=0)
+@pytest.mark.parametrize("steps", [11, 41])
+def test_1d_routes_match_oracle(vg_ctx, n, order, steps):
+    kw = dict(order=order, dim=1, dx=1.0 / n, cfl=0.7, tfinal=math.inf, max_steps=steps, bias=0.0, limiter=0)
     for bc in (S.TRANSMISSIVE, S.PERIODIC):
         w = _euler(n)
-        r = S.euler_solve(w, 1, 1.0 / n, 0.7, math.inf, order=order, limiter=0, max_steps=11, bc=bc)
+        r = S.euler_solve(w, 1, 1.0 / n, 0.7, math.inf, order=order, limiter=0, max_steps=steps, bc=bc)
         ref, dts = O.euler_solve(w, params=EULER, bc=bc, **kw)
         O.assert_bitwise(r.dt, dts, f"euler n {n} dt")
         O.assert_bitwise(r.cells, ref, f"euler n {n} state")
         w = _mhd(n)
-        r = S.mhd_solve(w, 1, 1.0 / n, 0.7, math.inf, order=order, limiter=0, max_steps=11, bc=bc,
+        r = S.mhd_solve(w, 1, 1.0 / n, 0.7, math.inf, order=order, limiter=0, max_steps=steps, bc=bc,
                         params=S.MHDMaterialParameters(5.0 / 3.0, 0.0, 0.7, 0.4))
         ref, dts = O.mhd_solve(w, gamma=5.0 / 3.0, ch=0.7, cp=0.4, bc=bc, **kw)
         O.assert_bitwise(r.dt, dts, f"mhd n {n} dt")
         O.assert_bitwise(r.cells, ref, f"mhd n {n} state")
 
 
-@pytest.mark.parametrize("n", [300, 700])
+@pytest.mark.parametrize("n", [300, 700, 2100])
 def test_final_time_and_caps_on_both_routes(vg_ctx, n):
     w = _euler(n)
     kw = dict(order=2, dim=1, dx=1.0 / n, cfl=0.8, bias=0.0, limiter=1, params=EULER)
@@ -59,9 +62,9 @@ def test_final_time_and_caps_on_both_routes(vg_ctx, n):
     assert r.stats.t == 0.05 and r.stats.steps == len(dts)
     O.assert_bitwise(r.dt, dts, "dt to the final time")
     O.assert_bitwise(r.cells, ref, "state at the final time")
-    for cap in (1, 8, 9, 23):
+    for cap in (1, 8, 9, 23, 33, 40, 47):
         r = S.euler_solve(w, 1, 1.0 / n, 0.8, 0.05, limiter=1, max_steps=cap)
-        assert r.stats.steps == cap
+        assert r.stats.steps == min(cap, len(dts))
         O.assert_bitwise(r.dt, dts[:cap], "capped dt prefix")
     assert S.euler_solve(w, 1, 1.0 / n, 0.8, 0.0, limiter=1).stats.steps == 0
 
@@ -86,3 +89,35 @@ def test_batch_widths_give_the_single_solves_bits(vg_ctx, n_inst, mode):
         one = S.mhd_solve(w[off[q]:off[q + 1]], 1, 1.0 / sizes[q], 0.6, 10.0, limiter=1, max_steps=7, mode=mode,
                           params=S.MHDMaterialParameters(5.0 / 3.0))
         O.assert_bitwise(r.cells[off[q]:off[q + 1]], one.cells, f"instance {q}")
+
+
+def _launches(ctx, w, t_final, max_steps, **kw):
+    """batch_solve launches of one Euler line: 1 where the whole solve is one workgroup's."""
+    ctx.reset_timing()
+    r = S.euler_solve(w, 1, 1.0 / len(w), 0.8, t_final, max_steps=max_steps, limiter=1, ctx=ctx, **kw)
+    return r, ctx.kernel_time("batch_solve")[0]
+
+
+def test_few_steps_of_a_longer_line_stay_in_one_workgroup():
+    """The grid path costs some tens of microseconds more a call, so by step cap or by
+    final time a short run of 509 to about 1500 cells is one launch; its result is the
+    long run's prefix either way."""
+    ctx = S.Context(0)
+    try:
+        ctx.set_timing(True)
+        for n, order in ((509, 2), (1016, 2), (1021, 1), (1530, 1)):
+            w = _euler(n)
+            long, launches = _launches(ctx, w, math.inf, 60, order=order)
+            assert launches == 0, (n, order)
+            short, launches = _launches(ctx, w, math.inf, 7, order=order)
+            assert launches == 1 and short.stats.steps == 7, (n, order)
+            O.assert_bitwise(short.dt, long.dt[:7], "capped dt")
+            # six steps of a fifth of a length and two whole ones
+            ended, launches = _launches(ctx, w, 0.999 * float(np.sum(long.dt[:8])), 0, order=order)
+            assert launches == 1 and ended.stats.steps == 8, (n, order)
+            O.assert_bitwise(ended.dt[:7], long.dt[:7], "dt to a final time")
+            # an infinite wave speed predicts no number of steps
+            w[n // 2, 0] = 0.0
+            assert _launches(ctx, w, 1.0, 60, order=order, raise_on_error=False)[1] == 0
+    finally:
+        ctx.close()

@@ -404,8 +404,8 @@ int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offse
     return VG_OK;
 }
 
-// Cells up to which one 1D solve runs as a batch of one: a workgroup that holds
-// the grid in one tile (FORCE, half the work: two) needs no launch per step.  Beyond
+// Cells up to which one 1D solve of any length runs as a batch of one: a workgroup that
+// holds the grid in one tile (FORCE, half the work: two) needs no launch per step.  Beyond
 // it the grid path spreads the line over the device, its step length taken inside
 // the sweep (sweep_x_begin_kernel): one launch a step.  Microseconds a step,
 // workgroup / grid path, EXACT: Euler SLIC 500 cells 5.4 / 6.1, 750 cells 10.5 /
@@ -417,15 +417,15 @@ int one_workgroup_1d(int order)
     return order == 2 ? BatchWidths<P>::wide - 4 : 2 * (BatchWidths<P>::wide - 2);
 }
 
-// One whole 1D solve by the faster route.  scan: the grid path also fills the
-// stats' count of inadmissible cells.
+// One whole 1D solve, as a batch of one or by the grid path.  scan: the grid path also
+// fills the stats' count of inadmissible cells.
 template <class P>
-int solve_line(vg_ctx *ctx, int order, int mode, const double *prim_in, double *prim_out, int n, double dx, double cfl,
-               double t_final, int max_steps, double bias, int limiter, int bc, const typename P::Params &m,
-               double *dt_log, int dt_cap, bool scan, vg_run_stats *stats)
+int solve_line(vg_ctx *ctx, bool one_workgroup, int order, int mode, const double *prim_in, double *prim_out, int n,
+               double dx, double cfl, double t_final, int max_steps, double bias, int limiter, int bc,
+               const typename P::Params &m, double *dt_log, int dt_cap, bool scan, vg_run_stats *stats)
 {
     const int64_t offsets[2] = {0, n};
-    if (n <= one_workgroup_1d<P>(order)) {
+    if (one_workgroup) {
         std::vector<typename P::Params> params(1, m);
         int32_t steps = 0;
         double tend = 0.0;
@@ -438,6 +438,17 @@ int solve_line(vg_ctx *ctx, int order, int mode, const double *prim_in, double *
     int rc = check_batch_args(order, mode, 1, offsets, prim_in, prim_out, &dx, &t_final, cfl, max_steps, bc);
     if (rc) return rc;
     GridState<P> g;
+    g.one_run = true;
+    if constexpr (!std::is_void_v<typename ReducedPhys<P>::type>) {
+        bool planar = true;
+        for (int i = 0; i < ReducedPhys<P>::kConst; i++)
+            for (int j = 0; j < n && planar; j++) {
+                unsigned long long b;
+                std::memcpy(&b, prim_in + (size_t)StoredFields<P>::n * j + ReducedPhys<P>::plane(i), sizeof(b));
+                planar = b == ReducedPhys<P>::bits(i);
+            }
+        g.host_planar = planar ? 1 : 0;
+    }
     rc = g.create(ctx, 1, 1, n);
     if (!rc) rc = g.load(prim_in, 0);
     if (!rc) rc = g.run(order, mode, dx, cfl, t_final, max_steps, bias, limiter, bc, m, dt_log, dt_cap, stats);

@@ -54,6 +54,33 @@ int check_run_args(int dim, int ny, int nx, double dx, double cfl, double t_fina
     return VG_OK;
 }
 
+// Whether a 1D solve runs as a batch of one: always where its one workgroup is the faster
+// route step for step, and a run of few steps also on a longer line, since the grid path
+// costs more a call.  By microseconds, the workgroup's a tile and step against the grid
+// path's extra a call and a step, its steps launched one by one or (from about 20) replayed
+// from a graph that has to be captured first.  Whole calls, workgroup / grid path: SLIC 750
+// cells 5 steps 220 / 249, 10 steps 272 / 289, 20 steps 376 / 368; FORCE 1021 cells 5 steps
+// 206 / 243, 20 steps 328 / 345, 50 steps 598 / 480.  The number of steps comes from the
+// initial state's wave speed and the first six steps' fifth of a length.
+bool line_in_one_workgroup(const double *prim, int n, double dx, double cfl, double t_final, int max_steps, int order,
+                           const vg_euler_params &mp)
+{
+    if (n <= vg::one_workgroup_1d<vg::EulerPhys>(order)) return true;
+    const int out = vg::BatchWidths<vg::EulerPhys>::wide - (order == 2 ? 4 : 2);
+    const double a_step = ((n + out - 1) / out) * (order == 2 ? 5.3 : 3.0);
+    auto faster = [&](double steps) { return a_step * steps <= std::min(20.0 + 9.0 * steps, 80.0 + 6.0 * steps); };
+    if (!faster(1.0)) return false;
+    if (max_steps > 0 && faster(max_steps)) return true;
+    if (!std::isfinite(t_final)) return false;
+    double S = 0.0;
+    for (int j = 0; j < n; j++) {
+        const double *w = prim + 6 * (size_t)j;
+        S = std::max(S, std::fabs(w[1]) + std::sqrt(mp.gamma * (w[4] + mp.p_inf) / w[0]));   // a NaN is passed over
+    }
+    const double steps = 5.0 + t_final * S / (cfl * dx);
+    return S > 0.0 && std::isfinite(steps) && faster(steps);
+}
+
 int solve(vg_ctx *ctx, int dim, const double *prim_in, double *prim_out, int ny, int nx, double dx, double cfl,
           double t_final, int max_steps, double bias, int limiter, int order, int bc, const vg_euler_params *mp,
           int mode, double *dt_log, int dt_log_cap, vg_run_stats *stats)
@@ -68,10 +95,12 @@ int solve(vg_ctx *ctx, int dim, const double *prim_in, double *prim_out, int ny,
     if (dim == 1) {
         vg_run_stats local{};
         local.first_nonfinite = -1;
-        const bool one_workgroup = nx <= vg::one_workgroup_1d<vg::EulerPhys>(order);
-        rc = vg::solve_line<vg::EulerPhys>(ctx, order, mode, prim_in, prim_out, nx, dx, cfl, t_final, max_steps, bias,
-                                           limiter, bc, to_params(mp), dt_log, dt_log_cap, true, &local);
-        for (int j = 0; one_workgroup && j < nx && rc == VG_OK; j++) {
+        const bool one_workgroup = line_in_one_workgroup(prim_in, nx, dx, cfl, t_final, max_steps, order, *mp);
+        // the scan of a short line takes the host less than the device's launch, copies and wait
+        const bool host_scan = one_workgroup || nx <= 2048;
+        rc = vg::solve_line<vg::EulerPhys>(ctx, one_workgroup, order, mode, prim_in, prim_out, nx, dx, cfl, t_final, max_steps, bias,
+                                           limiter, bc, to_params(mp), dt_log, dt_log_cap, !host_scan, &local);
+        for (int j = 0; host_scan && j < nx && rc == VG_OK; j++) {
             const double *w = prim_out + 6 * (size_t)j;
             bool bad = !(w[0] > 0.0) || !((w[4] + mp->p_inf) > 0.0);
             for (int f = 0; f < 6; f++) bad = bad || !std::isfinite(w[f]);

@@ -294,6 +294,8 @@ struct GridState {
     int y_variant = -1;            // y-sweep shape, autotuned per grid shape (-1: default_y)
     bool reduced = false;          // this run sweeps with ReducedPhys<P> (constant planes checked)
     bool planar_known = false;     // both buffers hold the constant planes (checked since the last load)
+    int host_planar = -1;          // the check's answer where the host has made it: 1 or 0 (-1: ask the device)
+    bool one_run = false;          // the grid serves one run only: a graph pays for itself in that run or not at all
     int *flag = nullptr;           // device flag of the constant-plane check (lazy)
     Clock *tune_clk = nullptr;     // scratch clock for tuning launches (lazy)
     Clock *sweep_clk = nullptr;    // scratch clock of the per-sweep entry points (lazy)
@@ -301,6 +303,10 @@ struct GridState {
     hipGraphExec_t graph = nullptr;  // captured chunk of steps
     std::string graph_key;           // arguments the graph was captured with
     static constexpr int kGraphSteps = 8;   // steps per captured chunk (even: buffers return to their start)
+    // A run of at most these captures nothing where one_run: a capture and its instantiation
+    // cost 65 us, a step launched one by one 3 us more (1500 cells, SLIC, 20 steps, a call:
+    // 430 us captured, 375 one by one).
+    static constexpr int kFewSteps = 32;
 
     int create(vg_ctx *c, int d, int y, int x)
     {
@@ -578,16 +584,18 @@ struct GridState {
                 reduced = true;
                 return VG_OK;
             }
-            if (!flag) VG_HIP(hipMalloc(&flag, sizeof(int)));
-            const int one = 1;
-            VG_HIP(hipMemcpyAsync(flag, &one, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-            constant_planes_kernel<ReducedPhys<P>><<<blocks_for(cells), 256, 0, ctx->stream>>>(buf[cur], plane, cells,
-                                                                                            flag);
-            int rc = launch_status("constant_planes");
-            if (rc) return rc;
-            int ok = 0;
-            VG_HIP(hipMemcpyAsync(&ok, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-            VG_HIP(hipStreamSynchronize(ctx->stream));
+            int ok = host_planar;
+            if (ok < 0) {
+                if (!flag) VG_HIP(hipMalloc(&flag, sizeof(int)));
+                const int one = 1;
+                VG_HIP(hipMemcpyAsync(flag, &one, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+                constant_planes_kernel<ReducedPhys<P>><<<blocks_for(cells), 256, 0, ctx->stream>>>(buf[cur], plane,
+                                                                                                cells, flag);
+                int rc = launch_status("constant_planes");
+                if (rc) return rc;
+                VG_HIP(hipMemcpyAsync(&ok, flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+                VG_HIP(hipStreamSynchronize(ctx->stream));
+            }
             if (!ok) return VG_OK;
             for (int i = 0; i < ReducedPhys<P>::kConst; i++) {
                 const long long off = (long long)ReducedPhys<P>::plane(i) * plane;
@@ -747,7 +755,8 @@ struct GridState {
         VG_HIP(hipEventCreate(&e1));
         VG_HIP(hipEventRecord(e0, ctx->stream));
         const int start_cur = cur;
-        int graph_steps = 0;   // steps enqueued as replays, before any one by one
+        // steps enqueued one by one before the first replay, and as replays
+        int first_steps = 0, graph_steps = 0;
         // Steps to enqueue before the clock is read again: what is left of the step
         // cap, and of the way to the final time at the last step's length (before
         // the start-up ramp is over, at the one its wave speed gives), so that few
@@ -817,6 +826,11 @@ struct GridState {
                     reps += 1;
                     rest = 0;
                 }
+                if (one_run && !graph && left <= kFewSteps) {
+                    reps = 0;
+                    rest = left;
+                }
+                if (graph_steps + reps == 0) first_steps += rest;
                 if (reps > 0) {
                     int rc = capture();
                     if (rc) return rc;
@@ -845,9 +859,11 @@ struct GridState {
                 if (max_steps > 0 && h.steps_this_run >= max_steps) break;
             }
         }
-        // a run that ended inside its replays may have left its keys in the second set
-        const bool two_sets = graph_steps >= h.steps_this_run && graph_steps > 0 && begins_in_sweep(ORDER, MODE, m);
-        clock_finish_kernel<<<1, 256, 0, ctx->stream>>>(clk, two_sets ? partials : nullptr, slots, n_partials);
+        // a run that ended inside its replays, after an odd number of their steps, left
+        // its keys in the second set
+        const int replayed = h.steps_this_run - first_steps;
+        const bool second = replayed > 0 && replayed <= graph_steps && (replayed & 1) && begins_in_sweep(ORDER, MODE, m);
+        clock_finish_kernel<<<1, 256, 0, ctx->stream>>>(clk, second ? partials : nullptr, slots, n_partials);
         int rc = launch_status("clock_finish");
         if (rc) return rc;
         VG_HIP(hipEventRecord(e1, ctx->stream));

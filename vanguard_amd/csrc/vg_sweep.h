@@ -547,13 +547,11 @@ static __global__ __launch_bounds__(kReduceThreads) void clock_begin_kernel(Cloc
     *c = h;
 }
 
-// End of a run: finishes its last step.  With `keys`, the run's steps began inside
-// their sweeps and left their wave-speed keys in two sets by turns: after an odd
-// number of steps the last keys, the second set's n, move to the first, where the
-// next run looks for them.
+// End of a run: finishes its last step.  With `keys`, the run's last wave-speed keys, n of
+// them, stand in the second set and move to the first, where the next run looks for them.
 static __global__ void clock_finish_kernel(Clock *c, unsigned long long *keys = nullptr, long long slots = 0, int n = 0)
 {
-    if (keys && (c->steps_this_run & 1))
+    if (keys)
         for (int k = threadIdx.x; k < n; k += blockDim.x) keys[k] = keys[slots + k];
     if (threadIdx.x == 0 && c->pending) {
         c->t += c->dt;
