@@ -2,6 +2,7 @@
 workgroup, at the sizes where the route or the width changes.  Add, multiply, divide
 and square root only: every comparison is bit for bit."""
 
+import ctypes
 import math
 
 import numpy as np
@@ -121,3 +122,20 @@ def test_few_steps_of_a_longer_line_stay_in_one_workgroup():
             assert _launches(ctx, w, 1.0, 60, order=order, raise_on_error=False)[1] == 0
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("n", [300, 5000])
+def test_a_rejected_call_leaves_the_run_statistics_alone(vg_ctx, n):
+    """An unknown mode: no step is taken, and of the caller's statistics only the step
+    counts and the time (MHD) are set."""
+    for nf, name in ((6, "vg_euler_solve_1d"), (9, "vg_mhd_solve_1d")):
+        w, out = np.ones((n, nf)), np.empty((n, nf))
+        st = _lib.RunStats(first_nonfinite=-1, nonfinite_cells=3, dt_min=0.25, dt_max=0.5, device_ms=1.5, wall_ms=2.5)
+        p = S.EulerMaterialParameters(1.4) if nf == 6 else S.MHDMaterialParameters(1.4)
+        sub = [] if nf == 6 else [0]
+        rc = getattr(vg_ctx.lib, name)(vg_ctx.handle, _lib.as_dptr(w), _lib.as_dptr(out), n, 1.0 / n, 0.5, 1.0, 5, 0.0,
+                                       0, 2, 0, *sub, ctypes.byref(p.c_struct()), 9, None, 0, ctypes.byref(st))
+        assert rc == _lib.VG_ERR_ARG
+        assert (st.first_nonfinite, st.nonfinite_cells) == (-1, 3), name
+        assert (st.dt_min, st.dt_max, st.device_ms, st.wall_ms) == (0.25, 0.5, 1.5, 2.5), name
+        assert st.steps == 0 and st.t == 0.0

@@ -435,6 +435,8 @@ int solve_line(vg_ctx *ctx, bool one_workgroup, int order, int mode, const doubl
         stats->t = tend;
         return rc;
     }
+    stats->steps = stats->total_steps = 0;
+    stats->t = 0.0;
     int rc = check_batch_args(order, mode, 1, offsets, prim_in, prim_out, &dx, &t_final, cfl, max_steps, bc);
     if (rc) return rc;
     GridState<P> g;
