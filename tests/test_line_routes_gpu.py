@@ -139,3 +139,14 @@ def test_a_rejected_call_leaves_the_run_statistics_alone(vg_ctx, n):
         assert (st.first_nonfinite, st.nonfinite_cells) == (-1, 3), name
         assert (st.dt_min, st.dt_max, st.device_ms, st.wall_ms) == (0.25, 0.5, 1.5, 2.5), name
         assert st.steps == 0 and st.t == 0.0
+
+
+def test_a_long_euler_line_that_cannot_advance_is_returned_as_it_is(vg_ctx):
+    """Euler lines of over 32,768 cells report a step that cannot advance t by their
+    statistics only: no steps, the initial state (finite and admissible here)."""
+    w = np.tile([1e-300, 0.0, 0.0, 0.0, 1e300, 1.0], (40000, 1))
+    r = S.euler_solve(w, 1, 1e-3, 0.8, 1.0)
+    assert r.status == _lib.VG_OK and r.stats.steps == 0 and r.stats.t == 0.0
+    O.assert_bitwise(r.cells, w, "state")
+    r = S.euler_solve(w[:32768], 1, 1e-3, 0.8, 1.0, raise_on_error=False)
+    assert r.status == _lib.VG_ERR_NONFINITE

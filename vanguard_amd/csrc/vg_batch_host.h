@@ -418,11 +418,13 @@ int one_workgroup_1d(int order)
 }
 
 // One whole 1D solve, as a batch of one or by the grid path.  scan: the grid path also
-// fills the stats' count of inadmissible cells.
+// fills the stats' count of inadmissible cells; report_stall: a step that cannot advance t
+// is an error there, as it is in a batch.
 template <class P>
 int solve_line(vg_ctx *ctx, bool one_workgroup, int order, int mode, const double *prim_in, double *prim_out, int n,
                double dx, double cfl, double t_final, int max_steps, double bias, int limiter, int bc,
-               const typename P::Params &m, double *dt_log, int dt_cap, bool scan, vg_run_stats *stats)
+               const typename P::Params &m, double *dt_log, int dt_cap, bool scan, bool report_stall,
+               vg_run_stats *stats)
 {
     const int64_t offsets[2] = {0, n};
     if (one_workgroup) {
@@ -455,7 +457,7 @@ int solve_line(vg_ctx *ctx, bool one_workgroup, int order, int mode, const doubl
     if (!rc) rc = g.load(prim_in, 0);
     if (!rc) rc = g.run(order, mode, dx, cfl, t_final, max_steps, bias, limiter, bc, m, dt_log, dt_cap, stats);
     if (!rc) rc = g.store(prim_out, 0);
-    if (!rc && g.stalled) {
+    if (!rc && g.stalled && report_stall) {
         set_error("1 instance(s) stopped because a time step could not advance t");
         rc = VG_ERR_NONFINITE;
     }

@@ -54,6 +54,10 @@ int check_run_args(int dim, int ny, int nx, double dx, double cfl, double t_fina
     return VG_OK;
 }
 
+// 1D solves of up to so many cells return VG_ERR_NONFINITE where a step cannot advance t;
+// longer ones, as 2D ones, return what they have, with the steps taken in the statistics.
+constexpr int kStallReported1D = 32768;
+
 // Whether a 1D solve runs as a batch of one: always where its one workgroup is the faster
 // route step for step, and a run of few steps also on a longer line, since the grid path
 // costs more a call.  By microseconds, the workgroup's a tile and step against the grid
@@ -99,7 +103,8 @@ int solve(vg_ctx *ctx, int dim, const double *prim_in, double *prim_out, int ny,
         // the scan of a short line takes the host less than the device's launch, copies and wait
         const bool host_scan = one_workgroup || nx <= 2048;
         rc = vg::solve_line<vg::EulerPhys>(ctx, one_workgroup, order, mode, prim_in, prim_out, nx, dx, cfl, t_final, max_steps, bias,
-                                           limiter, bc, to_params(mp), dt_log, dt_log_cap, !host_scan, &local);
+                                           limiter, bc, to_params(mp), dt_log, dt_log_cap, !host_scan,
+                                           nx <= kStallReported1D, &local);
         for (int j = 0; host_scan && j < nx && rc == VG_OK; j++) {
             const double *w = prim_out + 6 * (size_t)j;
             bool bad = !(w[0] > 0.0) || !((w[4] + mp->p_inf) > 0.0);

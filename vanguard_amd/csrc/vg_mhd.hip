@@ -72,7 +72,7 @@ int vg_mhd_solve_1d(vg_ctx *ctx, const double *prim_in, double *prim_out, int n,
     if (rc) return rc;
     vg_run_stats local = stats ? *stats : vg_run_stats{};   // a rejected call sets steps and time only
     rc = vg::solve_line<MHDPhys>(ctx, n <= vg::one_workgroup_1d<MHDPhys>(order), order, mode, prim_in, prim_out, n, dx, cfl, t_final, max_steps, bias, limiter, bc,
-                                 to_params(mp), dt_log, dt_log_cap, false, &local);
+                                 to_params(mp), dt_log, dt_log_cap, false, true, &local);
     if (stats) *stats = local;
     return rc;
 }
