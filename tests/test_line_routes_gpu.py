@@ -150,3 +150,24 @@ def test_a_long_euler_line_that_cannot_advance_is_returned_as_it_is(vg_ctx):
     O.assert_bitwise(r.cells, w, "state")
     r = S.euler_solve(w[:32768], 1, 1e-3, 0.8, 1.0, raise_on_error=False)
     assert r.status == _lib.VG_ERR_NONFINITE
+
+
+# Up to 256 instances take the limiter by selects, more by branches.
+@pytest.mark.parametrize("n_inst", [256, 257])
+@pytest.mark.parametrize("limiter,bias", [(0, 0.0), (1, -0.35), (2, 1.0), (1, 1.5)])
+def test_batches_on_both_sides_of_the_limiter_rule_match_oracle(vg_ctx, n_inst, limiter, bias):
+    sizes = 20 + (13 * np.arange(n_inst)) % 110
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    kw = dict(order=2, dim=1, cfl=0.6, tfinal=10.0, max_steps=7, bias=bias, limiter=limiter)
+    we = np.concatenate([_euler(int(n)) for n in sizes])
+    wm = np.concatenate([_mhd(int(n)) for n in sizes])
+    e = S.euler_solve_batch(we, off, 1.0 / sizes, [S.EulerMaterialParameters(*EULER)] * n_inst, np.full(n_inst, 10.0),
+                            0.6, max_steps=7, bias=bias, limiter=limiter)
+    m = S.mhd_solve_batch(wm, off, 1.0 / sizes, np.full(n_inst, 5.0 / 3.0), 10.0, 0.6, max_steps=7, bias=bias,
+                          limiter=limiter)
+    for q in range(0, n_inst, 32):
+        a, b = off[q], off[q + 1]
+        ref, _ = O.euler_solve(we[a:b], dx=1.0 / sizes[q], params=EULER, **kw)
+        O.assert_bitwise(e.cells[a:b], ref, f"euler instance {q}")
+        ref, _ = O.mhd_solve(wm[a:b], dx=1.0 / sizes[q], gamma=5.0 / 3.0, **kw)
+        O.assert_bitwise(m.cells[a:b], ref, f"mhd instance {q}")

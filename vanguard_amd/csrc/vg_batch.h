@@ -64,7 +64,7 @@ __device__ __forceinline__ unsigned long long block_allreduce_max(unsigned long 
 template <class P, int BS>
 constexpr int kBatchWaves = (P::NF >= 9 && BS <= 256) ? 3 : 1;
 
-template <class P, int ORDER, int MODE, int BS>
+template <class P, int ORDER, int MODE, int BS, bool BRANCHES>
 __global__ __launch_bounds__(BS, (kBatchWaves<P, BS>)) void batch_solve_kernel(BatchArgs<P> a)
 {
     constexpr int NF = P::NF;
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(BS, (kBatchWaves<P, BS>)) void batch_solve_kernel(B
             double w[NF];
             load_prim<NF>(A, n, jj, w);
             const unsigned long long k2 =
-                line_tile<P, 0, ORDER, MODE, BS, 1, false, false>(m, sc, a.bias, a.limiter, w, j < n, B, n, j, 1, true, s_a, s_e);
+                line_tile<P, 0, ORDER, MODE, BS, 1, BRANCHES, false>(m, sc, a.bias, a.limiter, w, j < n, B, n, j, 1, true, s_a, s_e);
             key = (k2 > key) ? k2 : key;
         }
         key = block_allreduce_max<BS>(key, s_red);   // its barriers also publish B for the next step

@@ -52,6 +52,14 @@ struct BatchBuffers {
 template <class P>
 struct BatchWidths;
 
+// Whether the EXACT SLIC batch kernel takes the limiter by branches: with more instances
+// than CUs, where it is bound by the instructions its waves issue and not by each one's
+// chain.  Microseconds a step, selects / branches, on flat shock tubes and on states with
+// waves everywhere: Euler 1000 x 300 cells 19.7 / 16.6 and 19.7 / 18.9, 5000 x 60 43.1 / 37.3
+// and 43.5 / 40.1; MHD 1000 x 500 40.3 / 33.0 and 42.0 / 42.4, 400 x 300 15.2 / 13.0 and 15.4
+// / 16.0; but MHD 64 x 250 5.7 / 5.4 and 5.5 / 6.2, Euler 3 x 100 4.1 / 4.1 and 4.0 / 4.4.
+inline bool batch_branches(int order, int mode, int n_inst) { return order == 2 && mode == VG_MODE_EXACT && n_inst > 256; }
+
 // f(std::integral_constant<int, BS>) for the width bs.
 template <class P, class F>
 auto with_batch_width(int bs, const F &f)
@@ -62,28 +70,32 @@ auto with_batch_width(int bs, const F &f)
     return f(std::integral_constant<int, W::narrow>{});
 }
 
-// f(std::integral_constant<int, ORDER>, std::integral_constant<int, MODE>)
+// f(std::integral_constant<int, ORDER>, std::integral_constant<int, MODE>,
+// std::bool_constant<BRANCHES>) for n_inst instances
 template <class F>
-auto with_order_mode(int order, int mode, const F &f)
+auto with_batch_kind(int order, int mode, int n_inst, const F &f)
 {
     using std::integral_constant;
-    if (order == 2)
-        return mode == VG_MODE_EXACT ? f(integral_constant<int, 2>{}, integral_constant<int, 0>{})
-                                     : f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
-    return mode == VG_MODE_EXACT ? f(integral_constant<int, 1>{}, integral_constant<int, 0>{})
-                                 : f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    if (order == 2 && mode == VG_MODE_EXACT)
+        return batch_branches(order, mode, n_inst)
+                   ? f(integral_constant<int, 2>{}, integral_constant<int, 0>{}, std::true_type{})
+                   : f(integral_constant<int, 2>{}, integral_constant<int, 0>{}, std::false_type{});
+    if (order == 2) return f(integral_constant<int, 2>{}, integral_constant<int, 1>{}, std::false_type{});
+    return mode == VG_MODE_EXACT ? f(integral_constant<int, 1>{}, integral_constant<int, 0>{}, std::false_type{})
+                                 : f(integral_constant<int, 1>{}, integral_constant<int, 1>{}, std::false_type{});
 }
 
 // Workgroups of the batch kernel resident at once on the device.
 template <class P>
-int batch_slots(vg_ctx *ctx, int order, int mode, int bs)
+int batch_slots(vg_ctx *ctx, int order, int mode, int n_inst, int bs)
 {
     int per_cu = 0, cus = 0;
-    const hipError_t e = with_order_mode(order, mode, [&](auto o, auto md) {
+    const hipError_t e = with_batch_kind(order, mode, n_inst, [&](auto o, auto md, auto br) {
         return with_batch_width<P>(bs, [&](auto w) {
             constexpr int BS = decltype(w)::value;
             return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, batch_solve_kernel<P, decltype(o)::value, decltype(md)::value, BS>, BS, 0);
+                &per_cu, batch_solve_kernel<P, decltype(o)::value, decltype(md)::value, BS, decltype(br)::value>, BS,
+                0);
         });
     });
     if (e != hipSuccess) per_cu = 1;
@@ -101,7 +113,7 @@ int batch_width(vg_ctx *ctx, int order, int mode, int n_inst, long long n_max)
     const int G = (order == 2) ? 2 : 1;
     int bs = W::narrow;
     for (int wider : {W::mid, W::wide})
-        if (n_max > bs - 2 * G && batch_slots<P>(ctx, order, mode, wider) >= n_inst) bs = wider;
+        if (n_max > bs - 2 * G && batch_slots<P>(ctx, order, mode, n_inst, wider) >= n_inst) bs = wider;
     return bs;
 }
 
@@ -109,10 +121,10 @@ template <class P>
 int launch_batch(vg_ctx *ctx, int order, int mode, int bs, const BatchArgs<P> &args, int n_inst)
 {
     return ctx->timed("batch_solve", [&] {
-        with_order_mode(order, mode, [&](auto o, auto md) {
+        with_batch_kind(order, mode, n_inst, [&](auto o, auto md, auto br) {
             with_batch_width<P>(bs, [&](auto w) {
                 constexpr int BS = decltype(w)::value;
-                batch_solve_kernel<P, decltype(o)::value, decltype(md)::value, BS>
+                batch_solve_kernel<P, decltype(o)::value, decltype(md)::value, BS, decltype(br)::value>
                     <<<n_inst, BS, 0, ctx->stream>>>(args);
             });
         });
@@ -224,7 +236,7 @@ int run_batch(vg_ctx *ctx, int order, int mode, int n_inst, const int64_t *offse
     // time the others finish instead of holding it alone on one CU.
     double budget = 0.0;
     if (n_inst > 1) {
-        const int slots = batch_slots<P>(ctx, order, mode, bs);
+        const int slots = batch_slots<P>(ctx, order, mode, n_inst, bs);
         if (n_inst > slots) {
             std::vector<double> sp(n_inst);
             VG_HIP(hipMemcpyAsync(sp.data(), b.speed, sizeof(double) * n_inst, hipMemcpyDeviceToHost, s));

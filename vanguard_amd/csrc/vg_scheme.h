@@ -251,16 +251,15 @@ __device__ __forceinline__ void with_divisors(double rho_l, double rho_r, bool a
     }
 }
 
-// FULL: for sweeps that fill the device (the walks of large grids), of which
-// evolve() takes the limiter's branches where there are few fields.
-template <class P, int DIR, int MODE, bool FULL = false>
+// BRANCHES: the EXACT limiter by branches (each lane's pieces only) instead of by selects
+// (every piece, the fields' chains side by side).  Branches for what fills the device with
+// few fields (the walks of large grids) or with many instances (the batch kernel).  EXACT x
+// walk of 4096 x 4096, 4 fields, branches / selects 367 / 383 us; one 200 x 200 tile sweep
+// 5.1 / 4.6 us; MHD 1024 x 1024 x tiles 67.7 / 61.9, y tiles 73.9 / 62.3; HPR 1024 x 1024 y
+// walk 183 / 164 us.
+template <class P, int DIR, int MODE, bool BRANCHES = false>
 struct Scheme {
     static constexpr int NF = P::NF;
-    // The limiter by branches (each lane's pieces only) or by selects (every piece,
-    // the fields' chains side by side).  EXACT x walk of 4096 x 4096, 4 fields, 367 us
-    // / 383; one 200 x 200 tile sweep 5.1 / 4.6 us; MHD 1024 x 1024 x tiles 67.7 / 61.9,
-    // y tiles 73.9 / 62.3; HPR 1024 x 1024 y walk 183 / 164 us.
-    static constexpr bool kLimiterBranches = FULL && NF <= 6;
     using Params = typename P::Params;
 
     __device__ static __forceinline__ void cons(const Params &m, const double (&w)[NF], double (&U)[NF])
@@ -305,7 +304,7 @@ struct Scheme {
         double xl[NF], xr[NF];
         const double cl = 0.5 * (1.0 + bias), cr = 0.5 * (1.0 - bias);
         if constexpr (MODE == MODE_EXACT) {
-            limited_sides<NF, kLimiterBranches ? 0 : (NF <= 9 ? NF : 3)>(UL, UM, UR, bias, limiter, xl, xr);
+            limited_sides<NF, BRANCHES ? 0 : (NF <= 9 ? NF : 3)>(UL, UM, UR, bias, limiter, xl, xr);
             double Fl[NF], Fr[NF];
             if constexpr (HasSharedDivisor<P>::value) {
                 // one branch for both sides, so their chains are scheduled together

@@ -93,7 +93,7 @@ __device__ __forceinline__ void block_max_to(unsigned long long *partials, unsig
 // the next tile.  s_a and s_e hold NF and 2 NF fields per thread; COMPACT (SLIC): NF
 // and NF, the left evolved states taking s_a's place once the cells' vectors have been
 // read, at two more barriers for a third less LDS.
-template <class P, int DIR, int ORDER, int MODE, int BS, int LW, bool FULL, bool COMPACT>
+template <class P, int DIR, int ORDER, int MODE, int BS, int LW, bool BRANCHES, bool COMPACT>
 __device__ __forceinline__ unsigned long long line_tile(const typename P::Params &m, const StepScalars &sc, double bias,
                                                         int limiter, const double (&w)[P::NF], bool write,
                                                         double *__restrict__ out, long long plane, long long out_idx,
@@ -103,7 +103,7 @@ __device__ __forceinline__ unsigned long long line_tile(const typename P::Params
     constexpr int G = (ORDER == 2) ? 2 : 1;
     constexpr int NP = BS / LW;
     constexpr bool kCompact = COMPACT && ORDER == 2;
-    using S = Scheme<P, DIR, MODE, FULL>;
+    using S = Scheme<P, DIR, MODE, BRANCHES>;
     const int tid = threadIdx.x, pos = tid / LW;
     double U[NF], Fp[NF];
     if (ORDER == 2) {
@@ -233,7 +233,7 @@ __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, d
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
     constexpr int OUT = BS - 2 * G;
-    constexpr bool FULL = RX > 1, COMPACT = !FULL && kCompactTile<P, ORDER, BS>;
+    constexpr bool WALK = RX > 1, BRANCHES = WALK && P::NF <= 6, COMPACT = !WALK && kCompactTile<P, ORDER, BS>;
     __shared__ double s_a[NF * BS];       // cell conserved vectors, later face fluxes
     // left evolved state (SLIC) / cell state (FORCE): U and F, or F only
     __shared__ double s_e[(COMPACT ? 1 : 2) * NF * BS];
@@ -250,7 +250,7 @@ __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, d
     const int i_begin = blockIdx.y * RX;
     unsigned long long key = 0;
     auto tile = [&](int i, const double(&w)[NF]) {
-        const unsigned long long k2 = line_tile<P, 0, ORDER, MODE, BS, 1, FULL, COMPACT>(
+        const unsigned long long k2 = line_tile<P, 0, ORDER, MODE, BS, 1, BRANCHES, COMPACT>(
             m, sc, a.bias, a.limiter, w, j < nx, a.out, a.plane, (long long)i * nx + j, a.dim, a.fuse_max != 0, s_a, s_e);
         key = (k2 > key) ? k2 : key;
     };
@@ -385,7 +385,7 @@ template <class P, int ORDER, int MODE, int BS, int H>
 __global__ __launch_bounds__(BS) void sweep_y_kernel(SweepArgs<P> a)
 {
     constexpr int NF = P::NF;
-    using S = Scheme<P, 1, MODE, true>;
+    using S = Scheme<P, 1, MODE, P::NF <= 6>;
 
     if (a.clk->done) return;
     const double ts = a.clk->dt * a.dt_scale;
