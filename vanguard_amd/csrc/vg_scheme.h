@@ -252,11 +252,12 @@ __device__ __forceinline__ void with_divisors(double rho_l, double rho_r, bool a
 }
 
 // BRANCHES: the EXACT limiter by branches (each lane's pieces only) instead of by selects
-// (every piece, the fields' chains side by side).  Branches for what fills the device with
-// few fields (the walks of large grids) or with many instances (the batch kernel).  EXACT x
-// walk of 4096 x 4096, 4 fields, branches / selects 367 / 383 us; one 200 x 200 tile sweep
-// 5.1 / 4.6 us; MHD 1024 x 1024 x tiles 67.7 / 61.9, y tiles 73.9 / 62.3; HPR 1024 x 1024 y
-// walk 183 / 164 us.
+// (every piece, the fields' chains side by side).  Branches for what fills the device:
+// the walks of large grids up to nine fields, the batch kernel with many instances.
+// EXACT, microseconds, branches / selects: 4 fields, x walk of 4096 x 4096 367 / 383, one
+// 200 x 200 tile sweep 5.1 / 4.6; MHD 1024 x 1024 x tiles 67.7 / 61.9, y tiles 73.9 / 62.3,
+// a step of 2300 x 2300 by walks 847 / 950 where one field varies, 1035 / 1071 where all
+// do; HPR 1024 x 1024 y walk 183 / 164.
 template <class P, int DIR, int MODE, bool BRANCHES = false>
 struct Scheme {
     static constexpr int NF = P::NF;

@@ -226,6 +226,10 @@ __device__ __forceinline__ bool clock_advance(Clock &c, unsigned long long mx)
 template <class P, int ORDER, int BS>
 constexpr bool kCompactTile = ORDER == 2 && (P::NF >= 9 || BS == kWave);
 
+// Whether walked sweeps take the limiter by branches (Scheme).
+template <class P>
+constexpr bool kWalkBranches = P::NF <= 9;
+
 // The rows of one x-sweep block, under time step dt and maximum wave speed S.
 template <class P, int ORDER, int MODE, int BS, int RX>
 __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, double S)
@@ -233,7 +237,8 @@ __device__ __forceinline__ void sweep_x_rows(const SweepArgs<P> &a, double dt, d
     constexpr int NF = P::NF;
     constexpr int G = (ORDER == 2) ? 2 : 1;
     constexpr int OUT = BS - 2 * G;
-    constexpr bool WALK = RX > 1, BRANCHES = WALK && P::NF <= 6, COMPACT = !WALK && kCompactTile<P, ORDER, BS>;
+    constexpr bool WALK = RX > 1, BRANCHES = WALK && kWalkBranches<P>;
+    constexpr bool COMPACT = !WALK && kCompactTile<P, ORDER, BS>;
     __shared__ double s_a[NF * BS];       // cell conserved vectors, later face fluxes
     // left evolved state (SLIC) / cell state (FORCE): U and F, or F only
     __shared__ double s_e[(COMPACT ? 1 : 2) * NF * BS];
@@ -385,7 +390,7 @@ template <class P, int ORDER, int MODE, int BS, int H>
 __global__ __launch_bounds__(BS) void sweep_y_kernel(SweepArgs<P> a)
 {
     constexpr int NF = P::NF;
-    using S = Scheme<P, 1, MODE, P::NF <= 6>;
+    using S = Scheme<P, 1, MODE, kWalkBranches<P>>;
 
     if (a.clk->done) return;
     const double ts = a.clk->dt * a.dt_scale;
