@@ -503,6 +503,8 @@ int vg_division_selfcheck(vg_ctx *ctx, int64_t n, const double *a, const double 
  * energy's division by (gamma - 1) rho, whose reciprocal comes from rho's). */
 int vg_scaled_division_selfcheck(vg_ctx *ctx, int64_t n, const double *a, const double *b, const double *c,
                                  double *scaled_q, double *ieee_q);
+/* The same for a / 3 (the HPR deviator's division of the Gramian's trace). */
+int vg_third_selfcheck(vg_ctx *ctx, int64_t n, const double *a, double *third_q, double *ieee_q);
 
 /* ---- two-material ideal MHD: real ghost fluid method ------------------- */
 

@@ -162,3 +162,21 @@ def test_quotients_by_a_scaled_density_are_ieee_division(scale):
                                               _lib.as_dptr(ieee))
     assert rc == 0
     assert_same(got, ieee, a, rho, f"scaled by {scale}")
+
+
+def test_thirds_are_ieee_division():
+    """a / 3 by the short sequence with RN(1 / 3): 2^-1000 to the largest double of either
+    sign, zeros, and numerators next to the midpoints of two neighbouring quotients."""
+    rng = np.random.default_rng(106)
+    q = make(rng, 200000, -998, 1021)
+    mid = (np.abs(q).view(np.uint64) & np.uint64((1 << 52) - 1)) | np.uint64(1 << 52)   # significands of 53 bits
+    # (q + half a unit) * 3 = (2 sig + 1) * 3 halves of a unit, and its neighbours
+    near = np.array([float(Fraction(3 * (2 * int(k) + 1), 2)) for k in mid[:50000]])
+    near = np.concatenate([near, np.nextafter(near, 0), np.nextafter(near, np.inf), 3.0 * mid[:50000].astype(np.float64)])
+    a = np.concatenate([make(rng, 1 << 22, -1000, 1023), near, -near, np.ldexp(near, -900), np.ldexp(near, 900), 3.0 * q,
+                        [0.0, -0.0, np.finfo(float).max, 2.0 ** -1000, 1.0, 3.0]])
+    a = a[np.isfinite(a) & ((np.abs(a) >= 2.0 ** -1000) | (a == 0))]
+    ctx = S.default_context()
+    got, ieee = np.empty_like(a), np.empty_like(a)
+    assert ctx.lib.vg_third_selfcheck(ctx.handle, a.size, _lib.as_dptr(a), _lib.as_dptr(got), _lib.as_dptr(ieee)) == 0
+    assert_same(got, ieee, a, np.full_like(a, 3.0), "third")

@@ -27,11 +27,15 @@
 //
 // Outside that range the shared form falls back to the IEEE division (a / b)
 // for divisors beyond 2^-100 <= b <= 2^100 (NaN, negative and other
-// densities).  Numerators are not checked: the tests show the short form
-// equal to the IEEE quotient for every numerator from 2^-1000 to 2^600 in
-// magnitude (and zero); below 2^-1000 (subnormal territory) it may be one
-// unit in the last place off, and above 2^600 it is not covered -- no
-// momentum or energy of a state the solvers reach.
+// densities).  Numerators are not checked -- momenta, energy, lambda, J (quot_group),
+// the pressure p + gamma p_inf (quot_scaled) and the trace of the distortion's Gramian
+// (third): the tests show the short form equal to the IEEE quotient for every numerator
+// from 2^-1000 to 2^600 in magnitude (and zero; the trace to its overflow); below 2^-1000
+// (subnormal territory) it may be one unit in the last place off, above 2^600 it is not
+// covered, and an infinite numerator gives a NaN where division gives an infinity: no
+// state the solvers reach.  An infinite energy or pressure makes the state's flux NaN
+// either way, since the flux divides the energy by rho; an infinite trace leaves NaN on
+// the deviator's diagonal, by division off it, and its norm and products NaN either way.
 //
 // The host build (used by tests/quotient_check.cpp) keeps y = RN(1 / b) and two
 // residual corrections, q = RN(a y), q += (a - b q) y twice, which Markstein's
@@ -141,7 +145,7 @@ __device__ __forceinline__ double quot_scaled(double a, const SharedDivisor &d, 
     return div_finish(a, b, y);
 }
 
-// RN(a / 3) for a zero or 2^-1000 <= |a| <= 2^1000 (a NaN for an infinite a).
+// RN(a / 3) for a zero or 2^-1000 <= |a| < 2^1024 (a NaN for an infinite a).
 __device__ __forceinline__ double third(double a) { return div_finish(a, 3.0, 1.0 / 3.0); }
 // Whether c is a scale quot_scaled takes.
 __device__ __forceinline__ bool scale_in_range(double c) { return (c >= 0x1p-20) && (c <= 0x1p+20); }

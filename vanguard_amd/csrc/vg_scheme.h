@@ -109,8 +109,8 @@ __device__ __forceinline__ void limited_slopes(const double (&num)[NF], const do
     }
 }
 
-// limited_sides with IEEE divisions, for operands out of the short ones' range: no
-// state the solvers reach.  The fields are a loop over copies in scratch memory, so
+// limited_sides with IEEE divisions, for operands out of the short ones' range (no state
+// the solvers reach) and for a bias outside [-1, 1], which they accept.  The fields are a loop over copies in scratch memory, so
 // that this path adds little code to the kernels of many fields.
 template <int NF, class NB>
 __device__ __forceinline__ void limited_sides_any_range(const NB &UL, const double (&UM)[NF], const NB &UR, double bias,

@@ -32,7 +32,42 @@ __global__ __launch_bounds__(256) void scaled_division_check_kernel(const double
     ieee_q[i] = x / (z * y);
 }
 
+__global__ __launch_bounds__(256) void third_check_kernel(const double *a, long long n, double *third_q, double *ieee_q)
+{
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    third_q[i] = vg::third(a[i]);
+    ieee_q[i] = a[i] / 3.0;
+}
+
 }  // namespace
+
+extern "C" int vg_third_selfcheck(vg_ctx *ctx, int64_t n, const double *a, double *third_q, double *ieee_q)
+{
+    vg::clear_error();
+    VG_CHECK(ctx != nullptr && a && third_q && ieee_q, "null argument");
+    VG_CHECK(n >= 1 && n <= (int64_t(1) << 26), "n must be in 1 .. 2^26");
+    int rc = vg::bind(ctx);
+    if (rc) return rc;
+    const size_t bytes = sizeof(double) * (size_t)n;
+    double *buf = nullptr;
+    VG_HIP(hipMalloc(&buf, 3 * bytes));
+    hipStream_t s = ctx->stream;
+    hipError_t e = hipMemcpyAsync(buf, a, bytes, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) {
+        third_check_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(buf, n, buf + n, buf + 2 * n);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(third_q, buf + n, bytes, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(ieee_q, buf + 2 * n, bytes, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    hipFree(buf);
+    if (e != hipSuccess) {
+        vg::set_error(std::string("vg_third_selfcheck: ") + hipGetErrorString(e));
+        return VG_ERR_HIP;
+    }
+    return VG_OK;
+}
 
 extern "C" int vg_scaled_division_selfcheck(vg_ctx *ctx, int64_t n, const double *a, const double *b, const double *c,
                                             double *scaled_q, double *ieee_q)
