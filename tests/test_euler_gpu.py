@@ -67,7 +67,7 @@ def test_fast_mode_within_tolerance(vg_ctx, name):
 
 
 @pytest.mark.parametrize("shape,bc,order,limiter,bias", [
-    ((37, 253), 0, 2, 0, 0.0),     # ragged: partial X tiles and Y segments
+    ((37, 253), 0, 2, 0, 0.0),     # ragged: partial tiles in x and y (walks: test_sweep_shapes_gpu.py)
     ((300, 7), 0, 2, 1, 0.25),
     ((5, 520), 1, 2, 2, -0.3),     # periodic, X tile wrap
     ((70, 66), 1, 1, 0, 0.0),      # periodic FORCE
