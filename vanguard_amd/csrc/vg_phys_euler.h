@@ -202,6 +202,22 @@ struct EulerPhys {
         F[4] = (U[4] + p) * vn;
         F[5] = U[5] * vn;
     }
+    // That flux less G.
+    template <int DIR>
+    __device__ static __forceinline__ void flux_less_fast(const Params &m, const double (&w)[NF], const double (&U)[NF],
+                                                          const double (&G)[NF], double (&D)[NF])
+    {
+#pragma clang fp contract(on)
+        (void)m;
+        const double vn = (DIR == 0) ? w[1] : w[2];
+        const double p = w[4];
+        D[0] = U[0] * vn - G[0];
+        D[1] = U[1] * vn + (DIR == 0 ? p - G[1] : -G[1]);
+        D[2] = U[2] * vn + (DIR == 1 ? p - G[2] : -G[2]);
+        D[3] = U[3] * vn - G[3];
+        D[4] = (U[4] + p) * vn - G[4];
+        D[5] = U[5] * vn - G[5];
+    }
 };
 
 // The same Euler state when its out-of-plane velocity is +0 and its reaction
@@ -337,6 +353,19 @@ struct EulerPlanarPhys {
         F[1] = U[1] * vn + (DIR == 0 ? p : 0.0);
         F[2] = U[2] * vn + (DIR == 1 ? p : 0.0);
         F[3] = (U[3] + p) * vn;
+    }
+    template <int DIR>
+    __device__ static __forceinline__ void flux_less_fast(const Params &m, const double (&w)[NF], const double (&U)[NF],
+                                                          const double (&G)[NF], double (&D)[NF])
+    {
+#pragma clang fp contract(on)
+        (void)m;
+        const double vn = (DIR == 0) ? w[1] : w[2];
+        const double p = w[3];
+        D[0] = U[0] * vn - G[0];
+        D[1] = U[1] * vn + (DIR == 0 ? p - G[1] : -G[1]);
+        D[2] = U[2] * vn + (DIR == 1 ? p - G[2] : -G[2]);
+        D[3] = (U[3] + p) * vn - G[3];
     }
 };
 

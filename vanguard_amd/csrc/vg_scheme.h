@@ -37,6 +37,18 @@ struct HasRoundTrip<P, decltype((void)&P::template round_trip<0>)> {
     static constexpr bool value = true;
 };
 
+// Physics whose FAST flux comes less another flux in the same expressions
+// (flux_less_fast), its products fused into the differences, as they are not across
+// statements (4096 x 4096, 4 fields: x walk 257 us a sweep without, 247 so).
+template <class P, class = void>
+struct HasFluxLess {
+    static constexpr bool value = false;
+};
+template <class P>
+struct HasFluxLess<P, decltype((void)&P::template flux_less_fast<0>)> {
+    static constexpr bool value = true;
+};
+
 // Correctly rounded division: the compiler's IEEE division, or the division
 // sequence without its scaling steps where the caller has shown the operands
 // in range (vg_quot.h).
@@ -336,13 +348,21 @@ struct Scheme {
                 xl[k] = UM[k] - (0.5 * d);
                 xr[k] = UM[k] + (0.5 * d);
             }
-            double Fl[NF], Fr[NF];
-            flux_of_cons(m, xl, Fl);
+            double D[NF], Fr[NF];
             flux_of_cons(m, xr, Fr);
+            if constexpr (HasFluxLess<P>::value) {
+                double w[NF];
+                P::cons_to_prim_fast(m, xl, w);
+                P::template flux_less_fast<DIR>(m, w, xl, Fr, D);
+            } else {
+                flux_of_cons(m, xl, D);
+#pragma unroll
+                for (int k = 0; k < NF; k++) D[k] = D[k] - Fr[k];
+            }
 #pragma unroll
             for (int k = 0; k < NF; k++) {
-                xl[k] = xl[k] + half_c * (Fl[k] - Fr[k]);
-                xr[k] = xr[k] + half_c * (Fl[k] - Fr[k]);
+                xl[k] = xl[k] + half_c * D[k];
+                xr[k] = xr[k] + half_c * D[k];
             }
         }
         if (MODE == MODE_EXACT) {
@@ -408,12 +428,12 @@ struct Scheme {
 #pragma clang fp contract(on)
 #pragma unroll
             for (int k = 0; k < NF; k++) {
-                lf[k] = 0.5 * ((a.F[k] + b.F[k]) + (lf_c * (a.U[k] - b.U[k])));
-                us[k] = 0.5 * ((a.U[k] + b.U[k]) + (ri_c * (a.F[k] - b.F[k])));
+                lf[k] = (a.F[k] + b.F[k]) + lf_c * (a.U[k] - b.U[k]);
+                us[k] = 0.5 * ((a.U[k] + b.U[k]) + ri_c * (a.F[k] - b.F[k]));
             }
             flux_of_cons(m, us, ri);
 #pragma unroll
-            for (int k = 0; k < NF; k++) F[k] = 0.5 * (lf[k] + ri[k]);
+            for (int k = 0; k < NF; k++) F[k] = 0.5 * (0.5 * lf[k] + ri[k]);   // the half fused into the sum
         }
     }
 
