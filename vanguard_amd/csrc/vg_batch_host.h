@@ -46,7 +46,7 @@ struct BatchBuffers {
 // Workgroup widths of the batch kernel: the narrowest keeps the most instances
 // resident, the wider ones give an instance more of its CU where there are fewer
 // instances than that (MHD, 256 - 2048 cells, 192 instances: 65.4 us a step at 128
-// threads, 25.8 at 512; 500 instances: 85.8 at 128, 52.0 at 256).  The tile's 3 NF
+// threads, 25.8 at 512; 500 instances, limiter by selects: 85.8 at 128, 52.0 at 256).  The tile's 3 NF
 // doubles per thread in LDS end the widening; 1024 threads of an Euler tile took
 // 8.7 us a step against 5.4 for 512.
 template <class P>
